@@ -101,6 +101,7 @@ void to_kernel_args(const fa_fwd_params* p, fa::KernelArgs* a) {
   a->split.n_merge = 0;
   a->split.xcd_heads = 0;
   a->split.pair = 0;
+  a->split.key_groups = 0;
   a->split.head_group = 0;
 }
 
@@ -266,12 +267,12 @@ fa_status fa_fwd_plan(const fa_fwd_params* p, int32_t compute_units, fa_fwd_plan
   fa::KernelArgs a;
   to_kernel_args(p, &a);
   out->workspace_bytes = fa::plan_split(a, compute_units, true, &a.split);
-  out->block_rows = fa::block_rows(a);
+  out->block_rows = a.split.key_groups ? 256 / a.split.key_groups : fa::block_rows(a);
   out->n_items = a.split.n_items;
   out->n_slots = a.split.n_slots;
   out->n_merge = a.split.n_merge;
   out->xcd_heads = a.split.xcd_heads;
-  out->key_halves = a.split.pair ? 2 : 1;
+  out->key_halves = a.split.pair ? 2 : a.split.key_groups == 4 ? 4 : 1;
   out->head_group = a.split.head_group;
   for (int i = 0; i < a.split.n_items; ++i) {
     const uint32_t info = a.split.item[i];

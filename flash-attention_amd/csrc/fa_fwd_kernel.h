@@ -30,6 +30,9 @@ struct SplitPlan {
   int32_t n_merge;   // q-tiles with more than one chunk (merged by the second kernel)
   int32_t xcd_heads; // > 0: XCD placement table over this many heads per XCD
   int32_t pair;      // 1: pair mode (8 waves per 128-row causal q-tile, no items)
+  // Key groups of a workgroup (fa_kg_kernel, no items): 4 on a 64-row q-tile,
+  // 2 on a 128-row non-causal one; else 0.
+  int32_t key_groups;
   // Causal grids in plain order with B*H a multiple of 8 (no items, no
   // table): each XCD runs its heads in groups of head_group, the q-tiles of
   // a group's heads interleaved longest first; 0 otherwise.
@@ -89,7 +92,8 @@ int block_rows(const KernelArgs& args);
 // Computes the work plan for args on a device with `compute_units` CUs
 // (host code, fa_plan.cpp).
 // Causal grids of 0.75 to 2 q-tiles per CU get pair mode (pair = 1, no
-// items, returns 0) with or without a workspace.  Otherwise, with
+// items, returns 0) and grids too small for the machine key groups
+// (key_groups, no items, returns 0), with or without a workspace.  Otherwise, with
 // allow_split it may choose split-KV and returns the workspace bytes it
 // needs; without (or when no split pays) it returns 0 and leaves either no
 // plan (n_items = 0) or an XCD placement table (xcd_heads > 0).

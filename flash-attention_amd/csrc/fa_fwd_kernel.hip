@@ -40,7 +40,9 @@
 //  * Pair mode (causal grids of 0.75 to 2 q-tiles of 128 rows per CU): 8
 //    waves run one q-tile, waves 0-3 on the even key tiles and waves 4-7 on
 //    the odd ones, each half with its own K/V ring; the halves meet in LDS
-//    at the end.  A long q-tile then never runs as a lone 4-wave workgroup
+//    at the end.  fa_kg_kernel is the same with four groups on 64-row
+//    q-tiles, or two on non-causal ones, for grids too small to put two waves
+//    on every SIMD (key_groups in fa_plan.cpp).  A long q-tile then never runs as a lone 4-wave workgroup
 //    on its CU (one wave per SIMD), which set the time of such grids.
 //  * O (and the fp32 split partials) leave through LDS: each wave parks its
 //    32-row tile in the then idle K/V ring and stores whole rows, 16
@@ -164,25 +166,31 @@ constexpr int kKWindow = 3;
 constexpr int kVWindow = 4;
 
 
+// The forward of one work item, shared by fa_fwd_kernel and fa_kg_kernel.
 // SPLIT: the grid runs the work items of args.split (chunks of q-tiles);
-// otherwise one workgroup per q-tile.  LSE_L (bf16 pair mode and split
+// otherwise one workgroup per q-tile.  LSE_L (bf16 key-group kernels and split
 // chunks, launches that write an LSE): the optimistic pass also keeps the
 // sums of the unrounded p, which only the LSE uses.
-template <int D, bool BF16, bool CAUSAL, int NW, bool SPLIT, bool PAIR = false, bool LSE_L = false>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    fa_fwd_kernel(const KernelArgs args) {
+template <int D, bool BF16, bool CAUSAL, int NW, bool SPLIT, int KG, bool LSE_L>
+__device__ __forceinline__ void fwd_body(const KernelArgs& args) {
   using T = Tile<D>;
   using Ops = ElemOps<BF16>;
-  // PAIR: 8 waves on one 128-row q-tile; waves 0-3 take the even key tiles
-  // of the item, waves 4-7 the odd ones, each half with its own K/V ring,
-  // and the halves are combined through LDS at the end.
-  static_assert(!PAIR || NW == 8, "pair mode runs 8 waves");
-  constexpr int BM = PAIR ? 128 : 32 * NW;
-  constexpr int NWD = PAIR ? 4 : NW;  // waves that stage one tile
-  constexpr int BN = T::BN;
+  // KG key groups (2: pair mode, 4): 8 waves on one q-tile of 32 * 8 / KG
+  // rows; group i (8 / KG waves) takes the key tiles i, i + KG, ... of the
+  // item with its own K/V ring, and the groups are combined through LDS at
+  // the end.
+  constexpr bool PAIR = KG > 1;
+  static_assert(!PAIR || (NW == 8 && !SPLIT), "key groups share 8 waves");
+  constexpr int BM = 32 * NW / KG;
+  constexpr int NWD = NW / KG;  // waves that stage one tile
+  // Keys per tile: 32 where four rings of 64-key tiles would not fit the LDS.
+  constexpr int BN = KG == 4 && D == 128 ? 32 : T::BN;
+  constexpr int NKB = BN / 32;             // 32-key blocks of a tile
+  constexpr int TILEB = BN * T::ROWB;      // bytes of a K or V tile
   constexpr int KSTEPS = D / 16;  // MFMA k-steps for S^T (k = head dim)
   constexpr int DBLK = D / 32;    // 32-wide head-dim blocks of O^T
-  constexpr int ITERS = T::BYTES / (1024 * NWD);  // DMA instructions per wave per tile
+  constexpr int ITERS = TILEB / (1024 * NWD);  // DMA instructions per wave per tile
+  constexpr int NWS = T::BYTES / (1024 * ITERS);  // dma_slot's waves per 64-key tile
   // Row sums of P in the per-tile checked pass.  O is always normalised by
   // the sum of the rounded P (the weights P V actually uses, so the weights
   // of a row sum to 1 and a dominant key's rounding cancels; with a lazy
@@ -241,11 +249,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
   // which keep v_dot2c.  The 8-wave and D = 64 kernels have no VGPRs left
   // for it next to kRescaleP.
   constexpr bool kMfmaNorm = kUnroundedSum && !kRescaleP && !SPLIT;
-  static_assert(ITERS >= 1 && T::BYTES % (1024 * NWD) == 0, "tile must split evenly over waves");
+  static_assert(ITERS >= 1 && TILEB % (1024 * NWD) == 0, "tile must split evenly over waves");
 
-  // LDS ring: K buffers 0/1 then V buffers 0/1 (pair mode: K 0/1 of each
-  // half, then V 0/1 of each half).
-  __shared__ __attribute__((aligned(1024))) char smem[(PAIR ? 8 : 4) * T::BYTES];
+  // LDS ring: K buffers 0/1 then V buffers 0/1 (key groups: K 0/1 of each
+  // group, then V 0/1 of each group).
+  __shared__ __attribute__((aligned(1024))) char smem[4 * KG * TILEB];
   // Set by any wave whose optimistic pass left a row with a non-finite sum.
   __shared__ int redo_flag;
   if (kMfmaSums && threadIdx.x == 0) redo_flag = 0;  // ordered by the first barrier
@@ -259,10 +267,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
   // B4 H32 N4096).  4-wave workgroups, whose SIMD partner belongs to another
   // workgroup, raise the priority only while issuing PV MFMAs (below).
   if (NW == 8 && wave >= 4) __builtin_amdgcn_s_setprio(1);
-  const int half = PAIR ? (wave >> 2) : 0;  // key-tile half (pair mode)
-  const int rw = PAIR ? (wave & 3) : wave;   // 32-row block of the q-tile
-  const int kslot = PAIR ? 2 * half : 0;     // this half's K ring slots
-  const int vslot = PAIR ? 4 + 2 * half : 2;  // and V ring slots
+  const int group = PAIR ? wave / NWD : 0;       // key group
+  const int rw = PAIR ? wave % NWD : wave;       // 32-row block of the q-tile
+  const int kslot = PAIR ? 2 * group : 0;        // this group's K ring slots
+  const int vslot = PAIR ? 2 * KG + 2 * group : 2;  // and V ring slots
   const int l32 = lane & 31;
   const int g = lane >> 5;         // which half of the wave
   const int lj = lane & 15;        // lane within its 16-lane group
@@ -329,20 +337,20 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
   // This item's key tiles [t_begin, t_end): chunk of n_chunks near-equal parts.
   const int t_begin = (int)((int64_t)chunk * q_tiles / n_chunks);
   const int t_end = (int)((int64_t)(chunk + 1) * q_tiles / n_chunks);
-  // This wave's tiles: t_first, t_first + TS, ... (pair mode: every other
-  // one), in n_steps steps shared by all waves of the workgroup.
-  constexpr int TS = PAIR ? 2 : 1;
-  const int t_first = t_begin + half;
-  const int n_steps = PAIR ? (t_end - t_begin + 1) / 2 : t_end - t_begin;
+  // This wave's tiles: t_first, t_first + KG, ... in n_steps steps shared by
+  // all waves of the workgroup.
+  constexpr int TS = KG;
+  const int t_first = t_begin + group;
+  const int n_steps = (t_end - t_begin + KG - 1) / KG;
 
   // ---- DMA plan: per-lane 32-bit source offsets within a tile ----
   uint32_t k_src[ITERS], v_src[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     int r, c;
-    dma_slot<D, NWD, false>(rw, it, lane, r, c);
+    dma_slot<D, NWS, false>(rw, it, lane, r, c);
     k_src[it] = (uint32_t)(r * ksb + c * 16);
-    dma_slot<D, NWD, true>(rw, it, lane, r, c);
+    dma_slot<D, NWS, true>(rw, it, lane, r, c);
     v_src[it] = (uint32_t)(r * vsb + c * 16);
   }
   const uint32_t smem_base = __builtin_amdgcn_readfirstlane(lds_addr(smem));
@@ -358,8 +366,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int row0 = t * BN;
     const char* kbase = kh + row0 * ksb;
     const char* vbase = vh + row0 * vsb;
-    const uint32_t kdst = wave_dma_base + (kslot + buf) * T::BYTES;
-    const uint32_t vdst = wave_dma_base + (vslot + buf) * T::BYTES;
+    const uint32_t kdst = wave_dma_base + (kslot + buf) * TILEB;
+    const uint32_t vdst = wave_dma_base + (vslot + buf) * TILEB;
     if constexpr (kLdsPoison) {
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
@@ -424,8 +432,38 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
               smem_base + q_lds + it * 1024);
     }
   }
+  // Key groups: the groups share their rows, so the workgroup stages each row
+  // once, the waves of a row block a part each (direct loads by every wave
+  // kept the address unit busy for 2000 cycles at D = 128).  The rows sit in
+  // K buffers 1, free until tile 1 is staged after the second barrier.
+  // (Waiting for K and Q first and for V only after the first S product
+  // measured 1...3 % slower at 4 key groups: its test stays in the tile loop.)
+  constexpr bool kShareQ = PAIR;
+  constexpr int QPS = TILEB / (32 * QRB);  // row blocks per ring slot
+  const uint32_t qs_lds =
+      (uint32_t)((2 * (rw / (QPS > 0 ? QPS : 1)) + 1) * TILEB + (rw % (QPS > 0 ? QPS : 1)) * 32 * QRB);
+  if constexpr (kShareQ) {
+    static_assert(!PAIR || (QPS >= 1 && (NWD + QPS - 1) / QPS <= KG && KSTEPS % KG == 0),
+                  "Q fits the K buffers 1");
+    constexpr int SH = KSTEPS / KG;  // 32 rows x QRB bytes = KSTEPS x 1 KiB
+    const int qr0 = min(wrow0, N - 1);
+    const char* qbase = qh + qr0 * qsb;
+#pragma unroll
+    for (int i = 0; i < SH; ++i) {
+      const int it = group * SH + i;
+      if constexpr (kLdsPoison) {
+        poison_kib(qs_lds + it * 1024);
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+      }
+      const int pos = it * 1024 + lane * 16;
+      const int r = pos / QRB, cs = (pos % QRB) / 16;
+      const int row = min(wrow0 + r, N - 1) - qr0;
+      dma_16b((uint32_t)(row * qsb + (cs ^ lds::row_swz(r, QRB)) * 16), qbase,
+              smem_base + qs_lds + it * 1024);
+    }
+  }
   i16x8 qf[KSTEPS];
-  if constexpr (!kStageQ) {
+  if constexpr (!kStageQ && !kShareQ) {
     const int qr = qrow < N ? qrow : N - 1;
     const char* qp = qh + qr * qsb + g * 16;
 #pragma unroll
@@ -456,7 +494,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
   uint32_t v_addr[DBLK];
 #pragma unroll
   for (int db = 0; db < DBLK; ++db)
-    v_addr[db] = smem_base + lds::v_read_offset<D>(0, 0, db, lane) + (vslot - 2) * T::BYTES;
+    v_addr[db] = smem_base + lds::v_read_offset<D>(0, 0, db, lane) + (vslot - 2) * TILEB;
 
   if constexpr (kStageQ) {
     // This wave's Q rows have landed (its own DMA): read the operands, and
@@ -470,6 +508,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
+  if constexpr (kShareQ) {
+#pragma unroll
+    for (int kk = 0; kk < KSTEPS; ++kk)
+      qf[kk] = *reinterpret_cast<const i16x8*>(smem + qs_lds +
+                                               lds::row_tile_offset(l32, 2 * kk + g, QRB));
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
 
   // OPT: the optimistic pass of kMfmaSums kernels (offset from the first
   // tile only, row sums on the matrix core); otherwise every tile checks its
@@ -479,35 +525,38 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     constexpr bool OPT = decltype(opt_c)::value;
     static_assert(!OPT || kMfmaSums, "the optimistic pass needs the matrix-core sums");
     const int kt0 = t * BN;
-    const char* kt = smem + (kslot + BUF) * T::BYTES;
+    const char* kt = smem + (kslot + BUF) * TILEB;
 
-    // ---- S^T = K Q^T : two 32-key blocks ----
+    // ---- S^T = K Q^T : NKB 32-key blocks ----
     // The K operands are read kKWindow k-steps ahead of their MFMA; the
     // sched_barriers keep the compiler from sinking each LDS read next to
     // its use (which would expose the full LDS latency on every MFMA).
-    f32x16 s[2];
+    f32x16 s[NKB];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[kb][i] = 0.0f;
     {
       constexpr int KD = kKWindow;
-      i16x8 ka[KD][2];
+      i16x8 ka[KD][NKB];
       static_for<0, KD>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         if constexpr (i < KSTEPS) {
-          ka[i][0] = *reinterpret_cast<const i16x8*>(kt + k_off[i]);
-          ka[i][1] = *reinterpret_cast<const i16x8*>(kt + 32 * T::ROWB + k_off[i]);
+#pragma unroll
+          for (int kb = 0; kb < NKB; ++kb)
+            ka[i][kb] = *reinterpret_cast<const i16x8*>(kt + kb * 32 * T::ROWB + k_off[i]);
         }
       });
       __builtin_amdgcn_sched_barrier(0);
       static_for<0, KSTEPS>([&](auto kk_c) {
         constexpr int kk = decltype(kk_c)::value;
-        s[0] = Ops::mfma(ka[kk % KD][0], qf[kk], s[0]);
-        s[1] = Ops::mfma(ka[kk % KD][1], qf[kk], s[1]);
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) s[kb] = Ops::mfma(ka[kk % KD][kb], qf[kk], s[kb]);
         if constexpr (kk + KD < KSTEPS) {
-          ka[kk % KD][0] = *reinterpret_cast<const i16x8*>(kt + k_off[kk + KD]);
-          ka[kk % KD][1] = *reinterpret_cast<const i16x8*>(kt + 32 * T::ROWB + k_off[kk + KD]);
+#pragma unroll
+          for (int kb = 0; kb < NKB; ++kb)
+            ka[kk % KD][kb] =
+                *reinterpret_cast<const i16x8*>(kt + kb * 32 * T::ROWB + k_off[kk + KD]);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -515,12 +564,12 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     // Prefetch the first kVWindow V^T operands: their LDS latency hides
     // behind the softmax.
     constexpr int VD = kVWindow;
-    constexpr int NPV = DBLK * 4;
+    constexpr int NPV = DBLK * 2 * NKB;
     i16x8 va[VD];
     static_for<0, VD>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
       constexpr int db = i % DBLK, ch = i / DBLK;
-      constexpr int off = (2 + BUF) * T::BYTES + ch * 16 * T::ROWB;
+      constexpr int off = (2 + BUF) * TILEB + ch * 16 * T::ROWB;
       va[i] = ds_read_tr_pair<off, off + 8 * T::ROWB>(v_addr[db]);
     });
     __builtin_amdgcn_sched_barrier(0);
@@ -534,7 +583,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
       // and a select per score.
       const int last = (CAUSAL ? min(N - 1, qrow) : N - 1) - kt0 - 4 * g;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int off = kb * 32 + 8 * (i >> 2) + (i & 3);
@@ -547,14 +596,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     // 8hh..8hh+7 of block kb.  t0/t1 sum this lane's even/odd keys.
     // pack(pval) packs the fp32 p given by pval(kb, i) and, in the checked
     // pass, sums them.
-    i16x8 pf[4];
+    i16x8 pf[2 * NKB];
     float t0, t1, tr;
     auto pack = [&](auto pval) FA_INLINE {
       t0 = 0.0f;
       t1 = 0.0f;
       tr = 0.0f;
 #pragma unroll
-      for (int ch = 0; ch < 4; ++ch) {
+      for (int ch = 0; ch < 2 * NKB; ++ch) {
         const int kb = ch >> 1, base = (ch & 1) * 8;
         u32x4 w;
 #pragma unroll
@@ -588,10 +637,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
       pack([&](int kb, int i) FA_INLINE { return fast_exp2(fmaf(s[kb][i], c, nmc)); });
     };
     // kRescaleP: p in fp32 (pv), kept past the check, packed by pack_pv.
-    float pv[2][16];
+    float pv[NKB][16];
     auto exp_f32 = [&](float nmc) FA_INLINE {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) pv[kb][i] = fast_exp2(fmaf(s[kb][i], c, nmc));
     };
@@ -624,14 +673,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     if (rederive) {
       // (In the optimistic pass this is the first tile: O and the sums are
       // still 0, so the rescale below is a no-op for them.)
-      const float mx = pair_max(max32(s[0], s[1]));
+      const float mx = pair_max(max32(s[0], s[NKB - 1]));
       if constexpr (OPT && !BF16) {
         // Spread test (kOptSpreadLimit) on the first tile, with the mean
         // estimated from 8 of the row's 64 keys (keys 4g, 4g+9, 4g+50,
-        // 4g+59 of each lane half): a wave that fails it asks the workgroup
+        // 4g+59 of each lane half; 32-key tiles: 4g, 4g+9, 4g+18, 4g+27): a wave that fails it asks the workgroup
         // to leave the optimistic pass after this tile.  -inf (masked)
         // scores make the mean -inf and fail it.
-        const float sm = (s[0][0] + s[0][5]) + (s[1][10] + s[1][15]);
+        const float sm = (s[0][0] + s[0][5]) + (s[NKB - 1][10] + s[NKB - 1][15]);
         const float mean = pair_sum(sm) * (1.0f / 8.0f);
         if (__any(!((mx - mean) * c <= kOptSpreadLimit)) && lane == 0) redo_flag = 1;
       }
@@ -670,7 +719,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
           exp_f32(none ? 0.0f : neg_mc);
         } else {
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
+          for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) pv[kb][i] *= alpha;
         }
@@ -694,7 +743,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         l_mfma = row_sum_mfma<BF16>(sum_sel, pf[ch], l_mfma);
       if constexpr (j + VD < NPV) {
         constexpr int db2 = (j + VD) % DBLK, ch2 = (j + VD) / DBLK;
-        constexpr int off = (2 + BUF) * T::BYTES + ch2 * 16 * T::ROWB;
+        constexpr int off = (2 + BUF) * TILEB + ch2 * 16 * T::ROWB;
         va[j % VD] = ds_read_tr_pair<off, off + 8 * T::ROWB>(v_addr[db2]);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -788,45 +837,80 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     lr_tot = lr_tot > 0.0f ? 1.0f : 0.0f;
   };
   if constexpr (PAIR) {
-    // Combine the halves: waves 4-7 hand O, the offset m and the sums
-    // (normalised as above) to their row partners through LDS, above the
-    // rows the epilogue stages; each half's terms are rescaled to the
-    // larger offset.
-    constexpr int XO = DBLK * 16 * 64;  // floats of O per wave
-    static_assert((XO + 4 * 64) * 4 % 1024 == 0 &&
-                      256 * D + 4 * (XO + 4 * 64) * 4 <= 8 * T::BYTES,
-                  "the combine area (whole KiB per wave) lies inside the ring");
-    float* xo = reinterpret_cast<float*>(smem + 256 * D) + rw * (XO + 4 * 64);
-    float* xm = xo + XO;
-    if (half == 1) {
+    // Combine the groups through the idle ring: every wave writes its
+    // normalised O (fp32 rows, CP head dims a pass) and its rows' (m, l, lr);
+    // then the KG waves of a row block finish 32 / KG of its rows each, 8
+    // head dims a lane, every group's term rescaled to the largest offset.
+    // (One group reading the others' whole O took 3200 cycles at D = 64 and
+    // 5200 at D = 128 with four groups.)
+    constexpr int RING = 4 * KG * TILEB;
+    constexpr int PASSES = NW * 32 * 4 * D + NW * 512 <= RING ? 1 : 2;
+    constexpr int CP = D / PASSES, ROWF = CP * 4;  // head dims, bytes of a row per pass
+    constexpr int LPR = CP / 8;                    // lanes per row
+    constexpr int FR = 32 / KG, RPI = 64 / LPR;    // rows to finish, rows per iteration
+    static_assert(NW * 32 * ROWF + NW * 512 <= RING && FR % RPI == 0 && DBLK % PASSES == 0,
+                  "the combine area lies inside the ring");
+    normalise_part();
+    char* const stats = smem + NW * 32 * ROWF;
+    char* const ot = smem + wave * 32 * ROWF;
+    static_for<0, PASSES>([&](auto p_c) {
+      constexpr int p = decltype(p_c)::value;
+      if (p > 0) __syncthreads();  // the reads of pass p - 1 are done
       if constexpr (kLdsPoison) {
-        const uint32_t off = (uint32_t)(reinterpret_cast<char*>(xo) - smem);
-        for (int kib = 0; kib < (XO + 4 * 64) * 4 / 1024; ++kib) poison_kib(off + kib * 1024);
+        for (int kib = 0; kib < ROWF / 32; ++kib) poison_kib(wave * 32 * ROWF + kib * 1024);
         __builtin_amdgcn_s_waitcnt(0xc07f);
       }
+      if (p == 0 && g == 0)
+        *reinterpret_cast<f32x4*>(stats + (wave * 32 + l32) * 16) = f32x4{m_run, l_tot, lr_tot, 0.0f};
 #pragma unroll
-      for (int db = 0; db < DBLK; ++db)
+      for (int b = 0; b < DBLK / PASSES; ++b)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) xo[(db * 16 + i) * 64 + lane] = o_acc[db][i];
-      *reinterpret_cast<f32x4*>(xm + 4 * lane) = f32x4{m_run, l_tot, lr_tot, 0.0f};
-    }
-    __syncthreads();
-    if (half == 1) return;
-    const f32x4 o1 = *reinterpret_cast<const f32x4*>(xm + 4 * lane);
-    const float inv1 = o1[2] > 0.0f ? 1.0f / o1[2] : 0.0f;
-    const float m1 = o1[2] > 0.0f ? o1[0] + __log2f(o1[2]) / c : -INFINITY;
-    normalise_part();
-    const float m = fmaxf(m_run, m1);
-    const float a0 = m_run == -INFINITY ? 0.0f : fast_exp2((m_run - m) * c);
-    const float a1 = m1 == -INFINITY ? 0.0f : fast_exp2((m1 - m) * c);
-    const float b0 = a0 * part_inv, b1 = a1 * inv1;
+        for (int r = 0; r < 4; ++r) {
+          const f32x16& o = o_acc[p * (DBLK / PASSES) + b];
+          *reinterpret_cast<f32x4*>(ot + lds::row_tile_offset(l32, 8 * b + 2 * r + g, ROWF)) =
+              f32x4{o[4 * r], o[4 * r + 1], o[4 * r + 2], o[4 * r + 3]} * part_inv;
+        }
+      __syncthreads();
 #pragma unroll
-    for (int db = 0; db < DBLK; ++db)
+      for (int it = 0; it < FR / RPI; ++it) {
+        const int r = group * FR + it * RPI + lane / LPR, cc = lane % LPR;
+        f32x4 st[KG], x[KG][2];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o_acc[db][i] = o_acc[db][i] * b0 + xo[(db * 16 + i) * 64 + lane] * b1;
-    l_tot = l_tot * a0 + o1[1] * b1;
-    lr_tot = lr_tot * a0 + (o1[2] > 0.0f ? a1 : 0.0f);
-    m_run = m;
+        for (int k = 0; k < KG; ++k) {
+          const int w = k * NWD + rw;
+          st[k] = *reinterpret_cast<const f32x4*>(stats + (w * 32 + r) * 16);
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            x[k][j] = *reinterpret_cast<const f32x4*>(
+                smem + w * 32 * ROWF + lds::row_tile_offset(r, 2 * cc + j, ROWF));
+        }
+        float m = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) m = fmaxf(m, st[k][0]);
+        f32x4 acc[2] = {};
+        float l = 0.0f, lr = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+          const float a = st[k][0] == -INFINITY ? 0.0f : fast_exp2((st[k][0] - m) * c);
+          l += a * st[k][1];
+          lr += a * st[k][2];
+          acc[0] += a * x[k][0];
+          acc[1] += a * x[k][1];
+        }
+        const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
+        const int q = wrow0 + r;
+        if (q < N) {
+          *reinterpret_cast<u32x4*>(oh + q * osb + (p * CP + 8 * cc) * 2) =
+              u32x4{pack2<BF16>(acc[0][0] * inv, acc[0][1] * inv),
+                    pack2<BF16>(acc[0][2] * inv, acc[0][3] * inv),
+                    pack2<BF16>(acc[1][0] * inv, acc[1][1] * inv),
+                    pack2<BF16>(acc[1][2] * inv, acc[1][3] * inv)};
+          if (p == 0 && cc == 0 && args.lse != nullptr)
+            args.lse[(int64_t)bh * N + q] = (m == -INFINITY ? 0.0f : m) * args.scale + __logf(l);
+        }
+      }
+    });
+    return;
   }
   const bool row_ok = qrow < N;
   // The output goes out through LDS, whole rows at a time.  In the O^T
@@ -931,6 +1015,25 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const float m_use = m_run == -INFINITY ? 0.0f : m_run;
     args.lse[(int64_t)bh * N + qrow] = m_use * args.scale + __logf(l_tot);
   }
+}
+
+// PAIR: pair mode, two key groups on a 128-row q-tile.
+template <int D, bool BF16, bool CAUSAL, int NW, bool SPLIT, bool PAIR = false, bool LSE_L = false>
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    fa_fwd_kernel(const KernelArgs args) {
+  fwd_body<D, BF16, CAUSAL, NW, SPLIT, PAIR ? 2 : 1, LSE_L>(args);
+}
+
+// Key groups outside pair mode: KG = 4 on a 64-row q-tile, KG = 2 on a
+// 128-row non-causal one.  What bounds such a launch is the length of one
+// workgroup: at 64 heads of rows on 256 CUs (B1 H8 N2048 D64 fp16, 256
+// workgroups) it spends 2.3 us before its first product (kernel arguments,
+// then 64 KiB of K, V and Q), 8 steps of 1.0 us and 1.2 us in the combine;
+// 25.6 us as split chunks with a merge launch, 13.5 us here.
+template <int D, bool BF16, bool CAUSAL, int KG, bool LSE_L>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    fa_kg_kernel(const KernelArgs args) {
+  fwd_body<D, BF16, CAUSAL, 8, false, KG, LSE_L>(args);
 }
 
 // Split-KV merge: one thread per 4 head-dim elements of a row of a q-tile
@@ -1055,6 +1158,22 @@ hipError_t launch_one(const KernelArgs& a, hipStream_t stream) {
   }
 }
 
+// Launch of fa_kg_kernel: one workgroup per 64-row q-tile, no items.
+template <int D, bool BF16, bool CAUSAL, int KG>
+hipError_t launch_kg(const KernelArgs& a, hipStream_t stream) {
+  if (a.split.n_items != 0) return hipErrorInvalidValue;
+  KernelArgs args = a;
+  constexpr int BM = 256 / KG;
+  args.n_qblocks = (args.seq_len + BM - 1) / BM;
+  const int64_t total = (int64_t)args.batch * args.heads * args.n_qblocks;
+  if (total > 0x7fffffff) return hipErrorInvalidValue;
+  void* kargs[] = {&args};
+  const void* fn = reinterpret_cast<const void*>(&fa_kg_kernel<D, BF16, CAUSAL, KG, false>);
+  if constexpr (BF16)
+    if (args.lse != nullptr) fn = reinterpret_cast<const void*>(&fa_kg_kernel<D, BF16, CAUSAL, KG, true>);
+  return hipLaunchKernel(fn, dim3((unsigned)total), dim3(512), kargs, 0, stream);
+}
+
 // The 16x16x32 MFMA kernel of every unsplit launch outside pair mode.
 #include "fa_fwd16.inc"
 
@@ -1087,6 +1206,10 @@ hipError_t launch_causal(const KernelArgs& a, hipStream_t stream) {
   // everywhere, for the counter comparison of the two shapes.
   const bool plain =
       a.split.n_items == 0 || (a.split.xcd_heads > 0 && a.split.n_merge == 0);
+  if (a.split.key_groups == 4)
+    return a.causal ? launch_kg<D, BF16, true, 4>(a, stream) : launch_kg<D, BF16, false, 4>(a, stream);
+  if (a.split.key_groups == 2)
+    return launch_kg<D, BF16, false, 2>(a, stream);
   if (a.causal) {
     // Long causal rows: 8-wave workgroups (fp16: +1.4 % at B1 H16 N16384,
     // +4 % with the matrix-core row sums they enable; bf16 only where the

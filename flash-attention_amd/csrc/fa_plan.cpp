@@ -38,12 +38,12 @@ int q_tile_tiles(const KernelArgs& a, int BM, int qb) {
   return (kv + kKeyTile - 1) / kKeyTile;
 }
 
-// Split-KV plan, or 0 items when no split pays (see plan_split).
-size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
+// Whether splitting key ranges pays on the grid of block_rows(a)-row q-tiles;
+// *total_tiles is its number of key tiles over all q-tiles.
+bool split_pays(const KernelArgs& a, int compute_units, double* total_tiles) {
   const int BM = block_rows(a);
   const int nq = (a.seq_len + BM - 1) / BM;
-  if (nq > kMaxSplitItems) return 0;
-  auto tiles = [&](int qb) { return q_tile_tiles(a, BM, qb); };
+  if (nq > kMaxSplitItems) return false;
   // Workgroup slots of the machine: two 4-wave workgroups or one 8-wave
   // workgroup per CU.  The unsplit grid finishes no earlier than its longest
   // q-tile (t_max key tiles) and no earlier than the total load over the
@@ -55,16 +55,26 @@ size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
   // and read of O per chunk, which ate the whole gain at B1 H16 N3000
   // causal (bound ratio 1.4) and left +11 % at H8 (2.8) and +50 % at
   // B1 H4 N8192 causal (3.9).
-  const int64_t slots = (int64_t)compute_units * (BM == 128 ? 2 : 1);
   int64_t sum = 0;
   int t_max = 0;
   for (int qb = 0; qb < nq; ++qb) {
-    sum += tiles(qb);
-    t_max = std::max(t_max, tiles(qb));
+    const int t = q_tile_tiles(a, BM, qb);
+    sum += t;
+    t_max = std::max(t_max, t);
   }
-  const double total = (double)sum * a.batch * a.heads;
-  const double bound = total / ((double)compute_units * (BM == 128 ? 1.1 : 1.0));
-  if (t_max <= 1.5 * bound + 8.0) return 0;
+  *total_tiles = (double)sum * a.batch * a.heads;
+  const double bound = *total_tiles / ((double)compute_units * (BM == 128 ? 1.1 : 1.0));
+  return t_max > 1.5 * bound + 8.0;
+}
+
+// Split-KV plan, or 0 items when no split pays (see plan_split).
+size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
+  double total = 0.0;
+  if (!split_pays(a, compute_units, &total)) return 0;
+  const int BM = block_rows(a);
+  const int nq = (a.seq_len + BM - 1) / BM;
+  auto tiles = [&](int qb) { return q_tile_tiles(a, BM, qb); };
+  const int64_t slots = (int64_t)compute_units * (BM == 128 ? 2 : 1);
   const double avg = total / (double)slots;  // per workgroup slot
   // Chunks of at most S key tiles, S about the average load (at least 8
   // tiles, so the per-item prologue and the partial write stay small).
@@ -199,17 +209,73 @@ int causal_head_group(const KernelArgs& a, int compute_units, bool pair) {
   if (g > 2 && hpx % 2 == 0 && 2 * nq >= 2 * slots_per_xcd) g = 2;
   return g;
 }
+
+// Key groups (fa_kg_kernel) for grids that leave CUs idle or with one wave per
+// SIMD: four groups on 64-row q-tiles while those fit one per CU, two on
+// 128-row q-tiles of non-causal problems while those do (causal ones are in
+// pair mode from 0.75 per CU on).  One workgroup of 8 waves then holds each
+// CU and a row's keys take a quarter (half) of the steps.  Past one
+// workgroup per CU the second round costs more than it saves (1.1 to 1.5
+// 128-row q-tiles per CU: 0.70...0.79 x).
+//
+// Measured us before -> after, fp16: four groups, B1 H8 N512 D64 8.7 -> 6.4,
+// H32 N512 D128 13.6 -> 9.4, H16 N1024 D64 14.1 -> 8.8, causal 16.3 -> 9.7,
+// H8 N2048 D64 25.6 -> 13.5, causal D128 27.1 -> 21.1; two groups, B2 H12
+// N1024 D128 22.0 -> 18.2, B1 H12 N2048 D64 39.5 -> 19.9, H6 N4096 D128
+// 85.2 -> 55.7.  Short rows: two key tiles gain from 4 groups on causal rows
+// (D = 64 6.7 -> 5.8, D = 128 8.3 -> 6.7) but not on D = 64 non-causal ones
+// (4.7 -> 5.0; four tiles 6.2 -> 5.7); at D = 128 they gain as well (7.4 ->
+// 6.4), but N = 128 non-causal is held to one 128-row q-tile per head by the
+// plan's tests, so the line is three tiles.  Two groups need 4 tiles at
+// D = 128 (10.4 -> 9.7) and 6 at D = 64 (4 tiles: 6.9 -> 7.1).
+//
+// Where split-KV would run (split_pays), its time is about constant plus the
+// work W per CU (128-row q-tiles x key tiles), that of four groups about
+// constant plus the row's T key tiles; the lines below cross where the
+// measured times do (e.g. D128 N2048: H2 and H3 non-causal T = 32 at the
+// line, causal H4 equal; N4096: H2 split 34.4 against 35.8 us, H4 four
+// groups 40.6 against 45.7).  Grids of at most an eighth (causal: a quarter)
+// of the CUs in 64-row q-tiles keep split-KV, whose chunks reach more CUs.
+// So do the few whose partials exceed the static scratch (D = 128, about 5
+// heads of N = 6000): fa_fwd_scratch refuses those, with or without key groups
+// for their neighbours.
+int key_groups(const KernelArgs& a, int compute_units) {
+  const int64_t bh = (int64_t)a.batch * a.heads;
+  const int T = (a.seq_len + kKeyTile - 1) / kKeyTile;
+  const int nq128 = (a.seq_len + 127) / 128;
+  const int64_t w64 = bh * T, w128 = bh * nq128;
+  const bool d64 = a.head_dim == 64, causal = a.causal != 0;
+  if (w64 > compute_units && (causal || w128 > compute_units)) return 0;
+  double total = 0.0;
+  const bool split = split_pays(a, compute_units, &total);
+  if (split) {
+    SplitPlan chunks;
+    if (plan_chunks(a, compute_units, &chunks) > kScratchBytes) return 0;
+  }
+  if (w64 <= compute_units) {
+    if (!split) return T >= (causal ? 2 : d64 ? 4 : 3) ? 4 : 0;
+    if (w64 <= compute_units / (causal ? 4 : 8)) return 0;
+    const double W = causal ? (double)bh * nq128 * (nq128 + 1) : (double)w128 * T;
+    const double t0 = causal ? (d64 ? 29.0 : 20.0) : (d64 ? 34.0 : 25.0);
+    const double per_w = causal ? 2.56 : (d64 ? 2.3 : 1.46);
+    return T < t0 + per_w * W / compute_units ? 4 : 0;
+  }
+  return T >= (d64 ? 6 : 4) ? 2 : 0;
+}
+
 }  // namespace
 
 size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, SplitPlan* plan) {
   plan->n_items = plan->n_slots = plan->n_merge = plan->xcd_heads = plan->pair = 0;
-  plan->head_group = 0;
+  plan->head_group = plan->key_groups = 0;
   if (compute_units < 1) return 0;
   if (pair_mode(a, compute_units)) {
     plan->pair = 1;
     plan->head_group = causal_head_group(a, compute_units, true);
     return 0;
   }
+  plan->key_groups = key_groups(a, compute_units);
+  if (plan->key_groups != 0) return 0;
   if (allow_split) {
     const size_t bytes = plan_chunks(a, compute_units, plan);
     if (bytes > 0) return bytes;

@@ -130,7 +130,9 @@ typedef struct {
   int32_t n_merge;          /* q-tiles with more than one chunk (merged by a second kernel) */
   int32_t xcd_heads;        /* > 0: XCD placement table (no split) over this many heads per XCD */
   int32_t key_halves;       /* 2: pair mode (8 waves per q-tile, each half on alternate key
-                               tiles, one workgroup per q-tile, no items); 1 otherwise */
+                               tiles, one workgroup per q-tile, no items); 4: the same with
+                               four key groups on 64-row q-tiles; 1 otherwise (two groups on
+                               the 128-row q-tiles of small non-causal grids included) */
   int32_t head_group;       /* > 0: causal grid without items, B*H a multiple of 8: each XCD
                                runs its heads in groups of this many, the q-tiles of a group
                                interleaved longest first; 0 otherwise */
