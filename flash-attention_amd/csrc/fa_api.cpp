@@ -90,7 +90,6 @@ void to_kernel_args(const fa_fwd_params* p, fa::KernelArgs* a) {
   a->head_dim = p->head_dim;
   a->causal = p->causal;
   a->bf16 = p->dtype == FA_DTYPE_BF16;
-  a->n_qblocks = 0;
   a->scale = p->softmax_scale;
   // c = scale * log2(e) (reference: src/config/config.cuh:84, forward_v6_mma.cuh:375)
   a->scale_log2 = p->softmax_scale * 1.4426950408889634f;

@@ -54,7 +54,16 @@ struct SplitPlan {
   uint32_t merge_slot[kMaxSplitItems];
 };
 
-struct KernelArgs {
+// n / d for n < 2^31 by a multiplication, d known on the host (fast_div).
+struct FastDiv {
+  uint32_t mul, shift;
+};
+
+// Arguments of the kernels without work items, all a kernel reads before its
+// first load: 216 bytes, where the plan's tables make 2.3 KB.  Every launch
+// copies its arguments to memory the GPU reads, and every workgroup starts by
+// waiting for them.
+struct FwdArgs {
   const void* q;
   const void* k;
   const void* v;
@@ -65,12 +74,22 @@ struct KernelArgs {
   int64_t k_stride_b, k_stride_h, k_stride_s;
   int64_t v_stride_b, v_stride_h, v_stride_s;
   int64_t o_stride_b, o_stride_h, o_stride_s;
-  int32_t batch, heads, seq_len, head_dim;
-  int32_t causal;
-  int32_t bf16;
-  int32_t n_qblocks;  // filled by the launcher
+  int32_t heads, seq_len;
   float scale;        // softmax scale (natural units, used for the LSE)
   float scale_log2;   // softmax scale * log2(e), used for exp2
+  // Order of the q-tiles in the grid, filled by the launcher (work_item).
+  int32_t n_qblocks;
+  int32_t per, tall;  // plain order: workgroups per XCD, XCDs with that many
+  int32_t hpx;        // > 0: whole heads per XCD (causal), in groups
+  int32_t group_heads, per_group;  // heads, q-tiles of a group
+  int32_t half;       // > 0: XCD placement table of 2 half q-tiles per XCD
+  FastDiv by_heads, by_qblocks, by_group, by_group_heads;
+};
+
+struct KernelArgs : FwdArgs {
+  int32_t batch, head_dim;
+  int32_t causal;
+  int32_t bf16;
   // Split-KV (filled by the launcher when a workspace is used).
   float* ws_o;        // [batch*heads][n_slots][BM][head_dim] fp32 partial O
   float* ws_ml;       // [batch*heads][n_slots][BM][4] fp32 (m, l, lr, unused)

@@ -166,13 +166,58 @@ constexpr int kKWindow = 3;
 constexpr int kVWindow = 4;
 
 
+// n / d for 0 <= n < 2^31 (make_fast_div).
+__device__ __forceinline__ int fast_div(int n, FastDiv d) {
+  return (int)(__umulhi(2u * (uint32_t)n, d.mul) >> d.shift);
+}
+
+// Head and q-tile of this workgroup in a grid without work items.
+//  * Causal, B * H a multiple of 8: whole heads per XCD, taken in groups of
+//    group_heads (the plan's choice; all of them if it does not divide their
+//    count): longest q-tiles first across a group's heads (interleaved),
+//    group after group.  XCD placement table (half > 0, one group): positions
+//    k and half + k of an XCD share a CU; the second half runs backwards, so
+//    each CU's q-tiles pair long with short.
+//  * Otherwise xcd_remap's order, causal q-tiles longest first.
+// The host passes the divisors' reciprocals: the divisions and the order
+// tables' loads were a quarter of the 1600...2900 cycles a workgroup spent
+// before its first load.
+//
+// TOGETHER: all of the arguments the prologue needs are loaded in one batch;
+// left to itself the compiler waits for the order's fields first and loads
+// the pointers and strides only then, a second trip to memory (B1 H2 N128 D64
+// 4.8 -> 4.5 us, causal B1 H8 N512 D64 6.8 -> 6.6).  Off in plain 8-wave
+// kernels, whose workgroups are long (B4 H32 N4096 -0.7 % with it).
+template <bool CAUSAL, bool TOGETHER>
+__device__ __forceinline__ void work_item(const FwdArgs& a, int& bh, int& qb) {
+  if constexpr (TOGETHER)
+    asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.q_stride_b), "s"(a.q_stride_h),
+                 "s"(a.q_stride_s), "s"(a.k_stride_b), "s"(a.k_stride_h), "s"(a.k_stride_s),
+                 "s"(a.v_stride_b), "s"(a.v_stride_h), "s"(a.v_stride_s), "s"(a.heads),
+                 "s"(a.seq_len), "s"(a.n_qblocks), "s"(a.by_heads.mul), "s"(a.by_heads.shift));
+  const int xcd = (int)(blockIdx.x & 7);
+  int i = (int)(blockIdx.x >> 3);
+  if (CAUSAL && a.hpx > 0) {
+    if (i >= a.half && a.half > 0) i = 3 * a.half - 1 - i;
+    const int grp = fast_div(i, a.by_group), w = i - grp * a.per_group;
+    const int wq = fast_div(w, a.by_group_heads);
+    bh = xcd * a.hpx + grp * a.group_heads + (w - wq * a.group_heads);
+    qb = a.n_qblocks - 1 - wq;
+  } else {
+    const int logical = xcd * a.per + i - max(xcd - a.tall, 0);
+    bh = fast_div(logical, a.by_qblocks);
+    const int item = logical - bh * a.n_qblocks;
+    qb = CAUSAL ? a.n_qblocks - 1 - item : item;
+  }
+}
+
 // The forward of one work item, shared by fa_fwd_kernel and fa_kg_kernel.
 // SPLIT: the grid runs the work items of args.split (chunks of q-tiles);
 // otherwise one workgroup per q-tile.  LSE_L (bf16 key-group kernels and split
 // chunks, launches that write an LSE): the optimistic pass also keeps the
 // sums of the unrounded p, which only the LSE uses.
 template <int D, bool BF16, bool CAUSAL, int NW, bool SPLIT, int KG, bool LSE_L>
-__device__ __forceinline__ void fwd_body(const KernelArgs& args) {
+__device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelArgs, FwdArgs>& args) {
   using T = Tile<D>;
   using Ops = ElemOps<BF16>;
   // KG key groups (2: pair mode, 4): 8 waves on one q-tile of 32 * 8 / KG
@@ -281,41 +326,25 @@ __device__ __forceinline__ void fwd_body(const KernelArgs& args) {
   // table: a chunk of a q-tile's key tiles (split-KV; the plan lists items
   // longest first), or the q-tile of this dispatch position within its XCD
   // (XCD placement table).
-  int bh, item;
-  if (SPLIT && args.split.xcd_heads > 0) {
-    // Hardware dispatch: workgroup b runs on XCD b % 8 as its (b / 8)-th.
-    item = (int)(blockIdx.x >> 3);
-    bh = (int)(blockIdx.x & 7) * args.split.xcd_heads + args.split.slot[item];
-  } else {
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int per_bh = SPLIT ? args.split.n_items : args.n_qblocks;
-    bh = logical / per_bh;
-    item = logical - bh * per_bh;
-  }
-  int qb, chunk = 0, n_chunks = 1;
+  int bh, qb, item = 0, chunk = 0, n_chunks = 1;
   if constexpr (SPLIT) {
+    if (args.split.xcd_heads > 0) {
+      // Hardware dispatch: workgroup b runs on XCD b % 8 as its (b / 8)-th.
+      item = (int)(blockIdx.x >> 3);
+      bh = (int)(blockIdx.x & 7) * args.split.xcd_heads + args.split.slot[item];
+    } else {
+      const int logical = xcd_remap(blockIdx.x, gridDim.x);
+      bh = logical / args.split.n_items;
+      item = logical - bh * args.split.n_items;
+    }
     const uint32_t info = args.split.item[item];
     qb = (int)(info & 0xffffu);
     chunk = (int)((info >> 16) & 0xffu);
     n_chunks = (int)(info >> 24);
   } else {
-    qb = CAUSAL ? args.n_qblocks - 1 - item : item;  // longest q-tiles first
-    if (CAUSAL && ((args.batch * args.heads) & 7) == 0) {
-      // Whole heads per XCD, taken in groups of args.split.head_group (the
-      // plan's choice; all of them if it does not divide their count):
-      // longest first across a group's heads (their q-tiles interleaved),
-      // group after group.  Same blocks per XCD as xcd_remap.
-      const int hpx = (args.batch * args.heads) >> 3;
-      const int hg = args.split.head_group;
-      const int grp_heads = hg > 0 && hpx % hg == 0 ? hg : hpx;
-      const int per_grp = grp_heads * args.n_qblocks;
-      const int i = (int)(blockIdx.x >> 3);
-      const int grp = i / per_grp, w = i - grp * per_grp;
-      bh = (int)(blockIdx.x & 7) * hpx + grp * grp_heads + w % grp_heads;
-      qb = args.n_qblocks - 1 - w / grp_heads;
-    }
+    work_item<CAUSAL, (NW == 4 || PAIR)>(args, bh, qb);
   }
-  const int b = bh / args.heads;
+  const int b = fast_div(bh, args.by_heads);
   const int h = bh - b * args.heads;
 
   const char* __restrict__ qh = reinterpret_cast<const char*>(args.q) +
@@ -948,7 +977,7 @@ __device__ __forceinline__ void fwd_body(const KernelArgs& args) {
   };
   const int wave_rows = max(0, min(32, N - wrow0));  // rows of this wave below N
 
-  if (SPLIT && n_chunks > 1) {
+  if constexpr (SPLIT) if (n_chunks > 1) {
     // ---- split-KV partial, normalised as above: O, offset m' (raw score
     // units; -inf when no key of this chunk is visible to the row), the row
     // sum l for the LSE and the sum of the rounded P (1, or 0 without keys)
@@ -1020,7 +1049,7 @@ __device__ __forceinline__ void fwd_body(const KernelArgs& args) {
 // PAIR: pair mode, two key groups on a 128-row q-tile.
 template <int D, bool BF16, bool CAUSAL, int NW, bool SPLIT, bool PAIR = false, bool LSE_L = false>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    fa_fwd_kernel(const KernelArgs args) {
+    fa_fwd_kernel(const std::conditional_t<SPLIT, KernelArgs, FwdArgs> args) {
   fwd_body<D, BF16, CAUSAL, NW, SPLIT, PAIR ? 2 : 1, LSE_L>(args);
 }
 
@@ -1032,7 +1061,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 // 25.6 us as split chunks with a merge launch, 13.5 us here.
 template <int D, bool BF16, bool CAUSAL, int KG, bool LSE_L>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    fa_kg_kernel(const KernelArgs args) {
+    fa_kg_kernel(const FwdArgs args) {
   fwd_body<D, BF16, CAUSAL, 8, false, KG, LSE_L>(args);
 }
 
@@ -1108,13 +1137,45 @@ __global__ void __launch_bounds__(256) fa_merge_kernel(const KernelArgs args, in
     args.lse[(int64_t)bh * args.seq_len + q] = (m == -INFINITY ? 0.0f : m) * args.scale + __logf(l);
 }
 
+FastDiv make_fast_div(uint32_t d) {
+  if (d < 1) d = 1;  // an unused divisor
+  uint32_t l = 0;    // ceil(log2 d)
+  while ((uint64_t(1) << l) < d) ++l;
+  // mul d = 2^(31 + l) + e with 0 < e <= d <= 2^l, so n mul / 2^(31 + l) =
+  // n / d + n e / (d 2^(31 + l)) is exact for n < 2^31 (the second term is
+  // below 1 / d); mul < 2^32 because d > 2^(l - 1).
+  return FastDiv{(uint32_t)((uint64_t(1) << (31 + l)) / d + 1), l};
+}
+
+// The grid order of q-tiles of BM rows (work_item) and its workgroup count.
+int64_t set_order(KernelArgs& a, int BM) {
+  const int bh = a.batch * a.heads;
+  a.n_qblocks = (a.seq_len + BM - 1) / BM;
+  const int64_t total = (int64_t)bh * a.n_qblocks;
+  a.per = (int)((total + 7) / 8);
+  a.tall = total % 8 == 0 ? 8 : (int)(total % 8);
+  a.hpx = a.causal && bh % 8 == 0 ? bh / 8 : 0;
+  a.half = 0;
+  a.group_heads = a.hpx;
+  if (a.split.xcd_heads > 0)
+    a.half = a.hpx * a.n_qblocks / 2;
+  else if (a.split.head_group > 0 && a.hpx % a.split.head_group == 0)
+    a.group_heads = a.split.head_group;
+  a.per_group = a.group_heads * a.n_qblocks;
+  a.by_heads = make_fast_div(a.heads);
+  a.by_qblocks = make_fast_div(a.n_qblocks);
+  a.by_group = make_fast_div(a.per_group);
+  a.by_group_heads = make_fast_div(a.group_heads);
+  return total;
+}
+
 template <int D, bool BF16, bool CAUSAL, int NW, bool PAIR = false>
 hipError_t launch_one(const KernelArgs& a, hipStream_t stream) {
   constexpr int BM = PAIR ? 128 : 32 * NW;
   KernelArgs args = a;
   // Pair mode runs one workgroup per q-tile, longest first; its plan has no items.
   if (PAIR && (a.split.n_items != 0 || !CAUSAL)) return hipErrorInvalidValue;
-  args.n_qblocks = (args.seq_len + BM - 1) / BM;
+  const int64_t qtiles = set_order(args, BM);
   // A plan is only valid for the block height it was made for; partials
   // need the workspace; a placement table covers 8 XCDs of whole heads.
   const int64_t bh = (int64_t)args.batch * args.heads;
@@ -1125,12 +1186,14 @@ hipError_t launch_one(const KernelArgs& a, hipStream_t stream) {
        (sp.xcd_heads > 0 && bh != 8 * (int64_t)sp.xcd_heads)))
     return hipErrorInvalidValue;
   const int64_t total = sp.xcd_heads > 0 ? 8 * (int64_t)sp.n_items
-                                         : (sp.n_items > 0 ? sp.n_items : args.n_qblocks) * bh;
+                        : sp.n_items > 0 ? sp.n_items * bh
+                                         : qtiles;
   if (total > 0x7fffffff) return hipErrorInvalidValue;
   // hipLaunchKernel returns this launch's own status: the thread's last-error
   // state is neither read nor cleared, so an earlier failure of an unrelated
   // HIP call by the caller is not reported as (or lost to) this launch.
   void* kargs[] = {&args};
+  void* fargs[] = {static_cast<FwdArgs*>(&args)};
   // bf16 pair and split launches that write an LSE: the LSE_L form, whose
   // optimistic pass keeps the unrounded sums.
   const bool lse_l = BF16 && args.lse != nullptr;
@@ -1138,7 +1201,7 @@ hipError_t launch_one(const KernelArgs& a, hipStream_t stream) {
     const void* fn = reinterpret_cast<const void*>(&fa_fwd_kernel<D, BF16, CAUSAL, NW, false, PAIR>);
     if constexpr (BF16 && PAIR)
       if (lse_l) fn = reinterpret_cast<const void*>(&fa_fwd_kernel<D, BF16, CAUSAL, NW, false, PAIR, true>);
-    return hipLaunchKernel(fn, dim3((unsigned)total), dim3(NW * 64), kargs, 0, stream);
+    return hipLaunchKernel(fn, dim3((unsigned)total), dim3(NW * 64), fargs, 0, stream);
   }
   if constexpr (PAIR) {
     return hipErrorInvalidValue;  // (rejected above: pair plans have no items)
@@ -1163,11 +1226,9 @@ template <int D, bool BF16, bool CAUSAL, int KG>
 hipError_t launch_kg(const KernelArgs& a, hipStream_t stream) {
   if (a.split.n_items != 0) return hipErrorInvalidValue;
   KernelArgs args = a;
-  constexpr int BM = 256 / KG;
-  args.n_qblocks = (args.seq_len + BM - 1) / BM;
-  const int64_t total = (int64_t)args.batch * args.heads * args.n_qblocks;
+  const int64_t total = set_order(args, 256 / KG);
   if (total > 0x7fffffff) return hipErrorInvalidValue;
-  void* kargs[] = {&args};
+  void* kargs[] = {static_cast<FwdArgs*>(&args)};
   const void* fn = reinterpret_cast<const void*>(&fa_kg_kernel<D, BF16, CAUSAL, KG, false>);
   if constexpr (BF16)
     if (args.lse != nullptr) fn = reinterpret_cast<const void*>(&fa_kg_kernel<D, BF16, CAUSAL, KG, true>);
