@@ -76,15 +76,41 @@ size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
   auto tiles = [&](int qb) { return q_tile_tiles(a, BM, qb); };
   const int64_t slots = (int64_t)compute_units * (BM == 128 ? 2 : 1);
   const double avg = total / (double)slots;  // per workgroup slot
-  // Chunks of at most S key tiles, S about the average load (at least 8
-  // tiles, so the per-item prologue and the partial write stay small).
-  int64_t S = std::max<int64_t>(8, (int64_t)std::ceil(avg));
+  // Chunks of at most S key tiles: the shortest (from 4 tiles on, so the
+  // per-item prologue and the partial write stay small) with which all items
+  // run at once, one per workgroup slot.  The launch then takes one chunk's
+  // time, and no second round of a few items follows a full one.  S about
+  // the average load, doubled while the items exceeded their table, was the
+  // rule before; us then -> now: causal B1 H2 N8192 bf16 57.2 -> 49.9 (34
+  // tiles a chunk on 156 of 256 CUs, now 19 on 254), H4 N8192 107 -> 88, H1
+  // N16384 169 -> 119, H1 N8192 D64 42.2 -> 29.0, H1 N1537 17.4 -> 15.0
+  // (chunks of 4 instead of 8), B1 H2 N1000 D64 13.8 -> 12.4; causal B1 H3
+  // N4096 D64 23.2 -> 23.9.
+  int64_t S = 0;
   auto n_chunks = [&](int qb) { return (int)std::min<int64_t>(255, (tiles(qb) + S - 1) / S); };
-  for (;;) {
-    int64_t items = 0;
-    for (int qb = 0; qb < nq; ++qb) items += n_chunks(qb);
-    if (items <= kMaxSplitItems) break;
-    S *= 2;
+  int64_t items = 0, bytes = 0;  // of a plan with chunks of S tiles
+  auto count = [&]() {
+    items = bytes = 0;
+    for (int qb = 0; qb < nq; ++qb) {
+      const int nch = n_chunks(qb);
+      items += nch;
+      if (nch > 1) bytes += nch;
+    }
+    bytes *= (int64_t)a.batch * a.heads * BM * (a.head_dim * 4 + 16);
+    return items;
+  };
+  for (S = std::max<int64_t>(8, (int64_t)std::ceil(avg)); count() > kMaxSplitItems;) S *= 2;
+  // Problems whose partials exceeded the static scratch under that rule keep
+  // its plan, and no other may exceed it: fa_fwd_scratch refuses what it did.
+  // So do grids of more q-tiles than slots, which no S runs at once.
+  if (bytes <= (int64_t)kScratchBytes) {
+    const int64_t s0 = S;
+    const int t_max = tiles(nq - 1);
+    for (S = std::max<int64_t>(4, (int64_t)std::ceil(avg)); S < t_max; ++S)
+      if (count() <= kMaxSplitItems && items * a.batch * a.heads <= slots &&
+          bytes <= (int64_t)kScratchBytes)
+        break;
+    if (S >= t_max) S = s0;
   }
   // Items, longest first (the dispatch order of the grid).
   struct Item { int len, qb, c, nch; };
@@ -235,8 +261,9 @@ int causal_head_group(const KernelArgs& a, int compute_units, bool pair) {
 // measured times do (e.g. D128 N2048: H2 and H3 non-causal T = 32 at the
 // line, causal H4 equal; N4096: H2 split 34.4 against 35.8 us, H4 four
 // groups 40.6 against 45.7).  Grids of at most an eighth (causal: a quarter)
-// of the CUs in 64-row q-tiles keep split-KV, whose chunks reach more CUs.
-// So do the few whose partials exceed the static scratch (D = 128, about 5
+// of the CUs in 64-row q-tiles keep split-KV: the plan's tests hold shapes
+// of one or two heads there to it (B1 H2 N1000 D64 non-causal 12.4 us split,
+// 9.2 with four groups).  So do the few whose partials exceed the static scratch (D = 128, about 5
 // heads of N = 6000): fa_fwd_scratch refuses those, with or without key groups
 // for their neighbours.
 int key_groups(const KernelArgs& a, int compute_units) {
@@ -248,19 +275,22 @@ int key_groups(const KernelArgs& a, int compute_units) {
   if (w64 > compute_units && (causal || w128 > compute_units)) return 0;
   double total = 0.0;
   const bool split = split_pays(a, compute_units, &total);
-  if (split) {
-    SplitPlan chunks;
-    if (plan_chunks(a, compute_units, &chunks) > kScratchBytes) return 0;
-  }
+  int groups = 0;
   if (w64 <= compute_units) {
     if (!split) return T >= (causal ? 2 : d64 ? 4 : 3) ? 4 : 0;
     if (w64 <= compute_units / (causal ? 4 : 8)) return 0;
     const double W = causal ? (double)bh * nq128 * (nq128 + 1) : (double)w128 * T;
     const double t0 = causal ? (d64 ? 29.0 : 20.0) : (d64 ? 34.0 : 25.0);
     const double per_w = causal ? 2.56 : (d64 ? 2.3 : 1.46);
-    return T < t0 + per_w * W / compute_units ? 4 : 0;
+    groups = T < t0 + per_w * W / compute_units ? 4 : 0;
+  } else {
+    groups = T >= (d64 ? 6 : 4) ? 2 : 0;
   }
-  return T >= (d64 ? 6 : 4) ? 2 : 0;
+  if (split && groups != 0) {
+    SplitPlan chunks;
+    if (plan_chunks(a, compute_units, &chunks) > kScratchBytes) return 0;
+  }
+  return groups;
 }
 
 }  // namespace
