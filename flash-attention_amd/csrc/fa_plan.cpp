@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <functional>
 
 #include "fa_fwd_kernel.h"
 
@@ -31,11 +32,19 @@ int block_rows(const KernelArgs& a) {
 namespace {
 
 constexpr int kKeyTile = 64;  // keys per K/V tile (Tile<D>::BN)
+constexpr int kMaxTiles = kMaxSplitItems * 256 / kKeyTile;  // key tiles of a row that may be split
+constexpr int kMaxCusPerXcd = 128;  // modelled (ChunkCost); an MI355X has 32
 
 // Key tiles of q-tile qb.
 int q_tile_tiles(const KernelArgs& a, int BM, int qb) {
   const int kv = a.causal ? std::min(a.seq_len, (qb + 1) * BM) : a.seq_len;
   return (kv + kKeyTile - 1) / kKeyTile;
+}
+
+// Workgroup slots of the machine: two 4-wave workgroups or one 8-wave
+// workgroup per CU.
+int64_t workgroup_slots(int BM, int compute_units) {
+  return (int64_t)compute_units * (BM == 128 ? 2 : 1);
 }
 
 // Whether splitting key ranges pays on the grid of block_rows(a)-row q-tiles;
@@ -44,17 +53,15 @@ bool split_pays(const KernelArgs& a, int compute_units, double* total_tiles) {
   const int BM = block_rows(a);
   const int nq = (a.seq_len + BM - 1) / BM;
   if (nq > kMaxSplitItems) return false;
-  // Workgroup slots of the machine: two 4-wave workgroups or one 8-wave
-  // workgroup per CU.  The unsplit grid finishes no earlier than its longest
-  // q-tile (t_max key tiles) and no earlier than the total load over the
-  // machine's throughput.  A CU running one 4-wave workgroup alone already
-  // reaches ~90 % of its two-workgroup throughput (measured: 1.14 us per
-  // 128x64 tile alone, 2.1 us each for two), so the throughput bound counts
-  // 1.1 workgroups per CU for 4-wave kernels.  Split only when the longest
-  // q-tile clearly dominates that bound: the partials cost an fp32 write
-  // and read of O per chunk, which ate the whole gain at B1 H16 N3000
-  // causal (bound ratio 1.4) and left +11 % at H8 (2.8) and +50 % at
-  // B1 H4 N8192 causal (3.9).
+  // The unsplit grid finishes no earlier than its longest q-tile (t_max key
+  // tiles) and no earlier than the total load over the machine's throughput.
+  // A CU running one 4-wave workgroup alone already reaches ~90 % of its
+  // two-workgroup throughput (measured: 1.14 us per 128x64 tile alone, 2.1 us
+  // each for two), so the throughput bound counts 1.1 workgroups per CU for
+  // 4-wave kernels.  Split only when the longest q-tile clearly dominates
+  // that bound: the partials cost an fp32 write and read of O per chunk,
+  // which ate the whole gain at B1 H16 N3000 causal (bound ratio 1.4) and
+  // left +11 % at H8 (2.8) and +50 % at B1 H4 N8192 causal (3.9).
   int64_t sum = 0;
   int t_max = 0;
   for (int qb = 0; qb < nq; ++qb) {
@@ -67,57 +74,199 @@ bool split_pays(const KernelArgs& a, int compute_units, double* total_tiles) {
   return t_max > 1.5 * bound + 8.0;
 }
 
-// Split-KV plan, or 0 items when no split pays (see plan_split).
-size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
+// Chunks of a split: at most S key tiles each (S = 0: no split).
+struct Chunks {
+  bool pays = false;  // split_pays
+  int average = 0;    // key tiles per workgroup slot
+  int S = 0;
+  int64_t bytes = 0;  // of the partials
+};
+
+// Chunks of q-tile qb.
+int q_tile_chunks(const KernelArgs& a, int BM, int qb, int S) {
+  return std::min(255, (q_tile_tiles(a, BM, qb) + S - 1) / S);
+}
+
+// Key tiles of chunk c of nch of a q-tile of T tiles (the kernel's t_begin and t_end).
+int chunk_tiles(int c, int nch, int T) {
+  return (int)((int64_t)(c + 1) * T / nch) - (int)((int64_t)c * T / nch);
+}
+
+// Items per (batch, head) with chunks of at most S tiles; *n_slots of them
+// leave partials.  Neither rises with S.
+int count_items(const KernelArgs& a, int BM, int nq, int S, int* n_slots) {
+  if (!a.causal) {  // every q-tile alike
+    const int nch = q_tile_chunks(a, BM, 0, S);
+    *n_slots = nch > 1 ? nq * nch : 0;
+    return nq * nch;
+  }
+  int items = 0;
+  *n_slots = 0;
+  for (int qb = 0; qb < nq; ++qb) {
+    const int nch = q_tile_chunks(a, BM, qb, S);
+    items += nch;
+    if (nch > 1) *n_slots += nch;
+  }
+  return items;
+}
+
+int64_t partial_bytes(const KernelArgs& a, int BM, int64_t n_slots) {
+  // Partial O (fp32) then (m, l, lr, unused) per row of every slot.
+  return (int64_t)a.batch * a.heads * n_slots * BM * (a.head_dim * 4 + 16);
+}
+
+// Modelled time of a split launch and its merge, in key tiles of a workgroup:
+// the last CU's load when each XCD hands out its run of items (head after
+// head, each longest first) to its CUs in order, + 10 per partial slot per CU
+// (written, read and merged) + 3/4 per four chunks of a row (the merge reads
+// four at a time).  Two 4-wave workgroups of a CU run at 1.1 times the rate of
+// one.  The constants are a fit to both rules' times on 1555 plans (H = 1...40,
+// N = 500...32700, both head dims and types): of the two it picks the slower
+// one by more than 2 % on 23 of them, by more than 5 % on 2 (both within the
+// spread of their own runs).
+struct ChunkCost {
+  const KernelArgs& a;
+  int compute_units, BM;
+  int lens[kMaxSplitItems], n = 0;  // items of a head, longest first
+  double partials;                  // the cost of the partials and the merge
+
+  ChunkCost(const KernelArgs& args, int cus, int bm, int nq, int S)
+      : a(args), compute_units(cus), BM(bm) {
+    // T tiles in nch chunks: T % nch of T / nch + 1 tiles, the rest of T / nch.
+    int count[kMaxTiles + 2] = {}, longest = 0, n_slots = 0;
+    const int distinct = a.causal ? nq : 1, alike = a.causal ? 1 : nq;
+    for (int qb = 0; qb < distinct; ++qb) {
+      const int T = q_tile_tiles(a, BM, qb), nch = q_tile_chunks(a, BM, qb, S);
+      const int len = T / nch, more = T - len * nch;
+      count[len + 1] += alike * more;
+      count[len] += alike * (nch - more);
+      longest = std::max(longest, len + (more > 0));
+      if (nch > 1) n_slots += alike * nch;
+    }
+    for (int l = longest; l > 0; --l)
+      for (int i = 0; i < count[l]; ++i) lens[n++] = l;
+    const int chunks = (q_tile_tiles(a, BM, nq - 1) + S - 1) / S;
+    partials = 10.0 * (double)n_slots * a.batch * a.heads / compute_units +
+               0.75 * ((chunks + 3) / 4);
+  }
+  int64_t items() const { return (int64_t)a.batch * a.heads * n; }
+  double rate() const { return BM == 128 && items() > compute_units ? 1.1 : 1.0; }
+  // No less than this, and exactly this with a CU for each item.
+  double least() const {
+    int64_t sum = 0;
+    for (int i = 0; i < n; ++i) sum += lens[i];
+    const double mean = (double)sum * a.batch * a.heads / compute_units / rate();
+    return partials + (items() <= compute_units ? lens[0] : std::max((double)lens[0], mean));
+  }
+  // The cost, or any value above `limit` once it is known to exceed that.
+  double cost(double limit = INFINITY) const {
+    if (items() <= compute_units || least() > limit) return least();
+    const int cpx = std::max(1, std::min(compute_units / 8, kMaxCusPerXcd));
+    const int64_t per = items() / 8, more = items() % 8;
+    int worst = 0, starts[8];
+    int64_t first = 0;
+    for (int x = 0; x < 8 && partials + worst / rate() <= limit; ++x) {
+      const int64_t count = per + (x < more ? 1 : 0);
+      int at = starts[x] = (int)(first % n);
+      first += count;
+      // XCDs whose run starts at the same item do alike (the first `more`
+      // XCDs, with an item more each, and the others apart).
+      const int* same = starts + (x < more ? 0 : more);
+      if (std::find(same, (const int*)starts + x, at) != starts + x) continue;
+      int cu[kMaxCusPerXcd];  // a heap of the CUs' loads, the least loaded first
+      for (int64_t i = 0; i < count; ++i) {
+        const int len = lens[at];
+        if (++at == n) at = 0;
+        if (i < cpx) {
+          cu[i] = len;
+          if (i == cpx - 1) std::make_heap(cu, cu + cpx, std::greater<int>());
+          worst = std::max(worst, len);
+          continue;
+        }
+        const int v = cu[0] + len;
+        int k = 0;  // v sinks from the root
+        for (int c = 1; c < cpx; c = 2 * k + 1) {
+          if (c + 1 < cpx && cu[c + 1] < cu[c]) ++c;
+          if (cu[c] >= v) break;
+          cu[k] = cu[c];
+          k = c;
+        }
+        cu[k] = v;
+        worst = std::max(worst, v);
+      }
+    }
+    return partials + std::max((double)lens[0], worst / rate());
+  }
+};
+
+// A split's chunks by the first rule of choose_chunks.
+Chunks average_chunks(const KernelArgs& a, int compute_units) {
+  Chunks ch;
   double total = 0.0;
-  if (!split_pays(a, compute_units, &total)) return 0;
+  ch.pays = split_pays(a, compute_units, &total);
+  if (!ch.pays) return ch;
   const int BM = block_rows(a);
   const int nq = (a.seq_len + BM - 1) / BM;
-  auto tiles = [&](int qb) { return q_tile_tiles(a, BM, qb); };
-  const int64_t slots = (int64_t)compute_units * (BM == 128 ? 2 : 1);
-  const double avg = total / (double)slots;  // per workgroup slot
-  // Chunks of at most S key tiles: the shortest (from 4 tiles on, so the
-  // per-item prologue and the partial write stay small) with which all items
-  // run at once, one per workgroup slot.  The launch then takes one chunk's
-  // time, and no second round of a few items follows a full one.  S about
-  // the average load, doubled while the items exceeded their table, was the
-  // rule before; us then -> now: causal B1 H2 N8192 bf16 57.2 -> 49.9 (34
-  // tiles a chunk on 156 of 256 CUs, now 19 on 254), H4 N8192 107 -> 88, H1
-  // N16384 169 -> 119, H1 N8192 D64 42.2 -> 29.0, H1 N1537 17.4 -> 15.0
-  // (chunks of 4 instead of 8), B1 H2 N1000 D64 13.8 -> 12.4; causal B1 H3
-  // N4096 D64 23.2 -> 23.9.
-  int64_t S = 0;
-  auto n_chunks = [&](int qb) { return (int)std::min<int64_t>(255, (tiles(qb) + S - 1) / S); };
-  int64_t items = 0, bytes = 0;  // of a plan with chunks of S tiles
-  auto count = [&]() {
-    items = bytes = 0;
-    for (int qb = 0; qb < nq; ++qb) {
-      const int nch = n_chunks(qb);
-      items += nch;
-      if (nch > 1) bytes += nch;
-    }
-    bytes *= (int64_t)a.batch * a.heads * BM * (a.head_dim * 4 + 16);
-    return items;
-  };
-  for (S = std::max<int64_t>(8, (int64_t)std::ceil(avg)); count() > kMaxSplitItems;) S *= 2;
-  // Problems whose partials exceeded the static scratch under that rule keep
-  // its plan, and no other may exceed it: fa_fwd_scratch refuses what it did.
+  ch.average = (int)std::ceil(total / (double)workgroup_slots(BM, compute_units));
+  int S = std::max(8, ch.average), n_slots = 0;
+  while (count_items(a, BM, nq, S, &n_slots) > kMaxSplitItems) S *= 2;
+  if (n_slots == 0) return ch;  // every q-tile whole
+  ch.S = S;
+  ch.bytes = partial_bytes(a, BM, n_slots);
+  return ch;
+}
+
+// The chunk length of a split, the better of two by ChunkCost:
+//  * about the average load of a workgroup slot (8 tiles at least), doubled
+//    while the items exceed their table (average_chunks);
+//  * the shortest (from 4 tiles on) with which all items run at once, one per
+//    slot: the launch takes one chunk's time, and no second round of a few
+//    items follows a full one.
+// us, first rule / second: causal B1 H2 N8192 D128 bf16 56.2 / 46.1 (34 tiles
+// a chunk on 156 of 256 CUs; 19 on 254), H1 N16384 169 / 119, H1 N8192 D64
+// 42.2 / 29.0.  But with nearly as many q-tiles as slots the second's chunks
+// are nearly whole q-tiles: fp16 D64 H5 N12000 146 / 166 (88 tiles, 172), H6
+// N10000 133 / 148; and where the first's items already run at once, one to a
+// CU, it only adds partials: H4 N2048 D128 20.9 / 23.4, H20 N1000 D64 16.7 /
+// 19.2.
+void choose_chunks(const KernelArgs& a, int compute_units, Chunks* ch) {
+  // Problems whose partials exceed the static scratch under the first rule
+  // keep its plan, and no other may exceed it: fa_fwd_scratch refuses them.
   // So do grids of more q-tiles than slots, which no S runs at once.
-  if (bytes <= (int64_t)kScratchBytes) {
-    const int64_t s0 = S;
-    const int t_max = tiles(nq - 1);
-    for (S = std::max<int64_t>(4, (int64_t)std::ceil(avg)); S < t_max; ++S)
-      if (count() <= kMaxSplitItems && items * a.batch * a.heads <= slots &&
-          bytes <= (int64_t)kScratchBytes)
-        break;
-    if (S >= t_max) S = s0;
-  }
+  const int BM = block_rows(a);
+  const int nq = (a.seq_len + BM - 1) / BM;
+  const int64_t bh = (int64_t)a.batch * a.heads;
+  const int64_t slots = workgroup_slots(BM, compute_units);
+  if (ch->bytes > (int64_t)kScratchBytes || nq * bh > slots) return;
+  const int t_max = q_tile_tiles(a, BM, nq - 1);
+  int lo = std::max(4, ch->average), n_slots = 0;
+  auto fits = [&](int S) {
+    const int items = count_items(a, BM, nq, S, &n_slots);
+    return items <= kMaxSplitItems && items * bh <= slots &&
+           partial_bytes(a, BM, n_slots) <= (int64_t)kScratchBytes;
+  };
+  while (lo < t_max && !fits(lo)) ++lo;
+  if (lo == t_max || lo == ch->S) return;
+  const ChunkCost c0(a, compute_units, BM, nq, ch->S), c1(a, compute_units, BM, nq, lo);
+  // The one with a CU for each item first: its cost needs no simulation.
+  const bool c0_first = c0.items() <= compute_units;
+  const double known = c0_first ? c0.cost() : c1.cost();
+  if (c0_first ? c1.cost(known) >= known : c0.cost(known) <= known) return;
+  count_items(a, BM, nq, lo, &n_slots);
+  ch->S = lo;
+  ch->bytes = partial_bytes(a, BM, n_slots);
+}
+
+// Fills the split-KV plan of chunks of at most S tiles.
+void plan_chunks(const KernelArgs& a, int S, SplitPlan* plan) {
+  const int BM = block_rows(a);
+  const int nq = (a.seq_len + BM - 1) / BM;
   // Items, longest first (the dispatch order of the grid).
   struct Item { int len, qb, c, nch; };
   Item list[kMaxSplitItems];
   int n = 0, slot_base[kMaxSplitItems], n_slots = 0, n_merge = 0;
   for (int qb = 0; qb < nq; ++qb) {
-    const int nch = n_chunks(qb), T = tiles(qb);
+    const int nch = q_tile_chunks(a, BM, qb, S), T = q_tile_tiles(a, BM, qb);
     slot_base[qb] = n_slots;
     if (nch > 1) {
       plan->merge[n_merge] = (uint32_t)qb | ((uint32_t)nch << 16);
@@ -125,13 +274,8 @@ size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
       ++n_merge;
       n_slots += nch;
     }
-    for (int c = 0; c < nch; ++c) {
-      // Same split of [0, T) as the kernel's t_begin / t_end.
-      const int len = (int)((int64_t)(c + 1) * T / nch) - (int)((int64_t)c * T / nch);
-      list[n++] = Item{len, qb, c, nch};
-    }
+    for (int c = 0; c < nch; ++c) list[n++] = Item{chunk_tiles(c, nch, T), qb, c, nch};
   }
-  if (n_merge == 0) return 0;
   std::stable_sort(list, list + n, [](const Item& x, const Item& y) {
     return x.len != y.len ? x.len > y.len : x.qb > y.qb;
   });
@@ -143,8 +287,6 @@ size_t plan_chunks(const KernelArgs& a, int compute_units, SplitPlan* plan) {
   plan->n_items = n;
   plan->n_slots = n_slots;
   plan->n_merge = n_merge;
-  // Partial O (fp32) then (m, l, lr, unused) per row of every slot.
-  return (size_t)a.batch * a.heads * n_slots * BM * ((size_t)a.head_dim * 4 + 16);
 }
 
 // XCD placement table for a causal 4-wave grid of one round: each XCD
@@ -266,18 +408,17 @@ int causal_head_group(const KernelArgs& a, int compute_units, bool pair) {
 // 9.2 with four groups).  So do the few whose partials exceed the static scratch (D = 128, about 5
 // heads of N = 6000): fa_fwd_scratch refuses those, with or without key groups
 // for their neighbours.
-int key_groups(const KernelArgs& a, int compute_units) {
+// ch: average_chunks.
+int key_groups(const KernelArgs& a, int compute_units, const Chunks& ch) {
   const int64_t bh = (int64_t)a.batch * a.heads;
   const int T = (a.seq_len + kKeyTile - 1) / kKeyTile;
   const int nq128 = (a.seq_len + 127) / 128;
   const int64_t w64 = bh * T, w128 = bh * nq128;
   const bool d64 = a.head_dim == 64, causal = a.causal != 0;
   if (w64 > compute_units && (causal || w128 > compute_units)) return 0;
-  double total = 0.0;
-  const bool split = split_pays(a, compute_units, &total);
   int groups = 0;
   if (w64 <= compute_units) {
-    if (!split) return T >= (causal ? 2 : d64 ? 4 : 3) ? 4 : 0;
+    if (!ch.pays) return T >= (causal ? 2 : d64 ? 4 : 3) ? 4 : 0;
     if (w64 <= compute_units / (causal ? 4 : 8)) return 0;
     const double W = causal ? (double)bh * nq128 * (nq128 + 1) : (double)w128 * T;
     const double t0 = causal ? (d64 ? 29.0 : 20.0) : (d64 ? 34.0 : 25.0);
@@ -286,10 +427,7 @@ int key_groups(const KernelArgs& a, int compute_units) {
   } else {
     groups = T >= (d64 ? 6 : 4) ? 2 : 0;
   }
-  if (split && groups != 0) {
-    SplitPlan chunks;
-    if (plan_chunks(a, compute_units, &chunks) > kScratchBytes) return 0;
-  }
+  if (ch.pays && groups != 0 && ch.bytes > (int64_t)kScratchBytes) return 0;
   return groups;
 }
 
@@ -304,12 +442,13 @@ size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, Spli
     plan->head_group = causal_head_group(a, compute_units, true);
     return 0;
   }
-  plan->key_groups = key_groups(a, compute_units);
+  Chunks ch = average_chunks(a, compute_units);
+  plan->key_groups = key_groups(a, compute_units, ch);
   if (plan->key_groups != 0) return 0;
-  if (allow_split) {
-    const size_t bytes = plan_chunks(a, compute_units, plan);
-    if (bytes > 0) return bytes;
-    plan->n_items = plan->n_slots = plan->n_merge = 0;
+  if (allow_split && ch.S > 0) {
+    choose_chunks(a, compute_units, &ch);
+    plan_chunks(a, ch.S, plan);
+    return (size_t)ch.bytes;
   }
   const size_t bytes = plan_xcd_table(a, compute_units, plan);
   if (plan->n_items == 0) plan->head_group = causal_head_group(a, compute_units, false);
