@@ -238,14 +238,18 @@ void choose_chunks(const KernelArgs& a, int compute_units, Chunks* ch) {
   const int64_t bh = (int64_t)a.batch * a.heads;
   const int64_t slots = workgroup_slots(BM, compute_units);
   if (ch->bytes > (int64_t)kScratchBytes || nq * bh > slots) return;
+  // The items, the slots and so the bytes fall as S rises: bisection.
   const int t_max = q_tile_tiles(a, BM, nq - 1);
-  int lo = std::max(4, ch->average), n_slots = 0;
+  int lo = std::max(4, ch->average), hi = t_max, n_slots = 0;
   auto fits = [&](int S) {
     const int items = count_items(a, BM, nq, S, &n_slots);
     return items <= kMaxSplitItems && items * bh <= slots &&
            partial_bytes(a, BM, n_slots) <= (int64_t)kScratchBytes;
   };
-  while (lo < t_max && !fits(lo)) ++lo;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (fits(mid)) hi = mid; else lo = mid + 1;
+  }
   if (lo == t_max || lo == ch->S) return;
   const ChunkCost c0(a, compute_units, BM, nq, ch->S), c1(a, compute_units, BM, nq, lo);
   // The one with a CU for each item first: its cost needs no simulation.

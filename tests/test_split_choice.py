@@ -116,3 +116,25 @@ def test_shorter_launch_is_taken(lib, D, causal):
                     assert mine.cost <= other.cost, (H, N, mine.cost, other.cost)
                     took.add(mine is first)
     assert took == {True, False} or not causal
+
+
+@pytest.mark.parametrize("H,N,D,causal", [
+    (1, 32512, 128, 1), (1, 28000, 64, 1), (1, 24000, 128, 1), (2, 24000, 64, 1), (4, 16384, 64, 1),
+    (1, 16384, 128, 1), (7, 2500, 128, 1), (8, 2048, 64, 1), (1, 16384, 128, 0),
+])
+def test_plan_time(lib, H, N, D, causal):
+    """The plan is made two or three times a call: about 10 us at most where
+    one without a split takes 1 (a search over every length took 27 to 130 us
+    for most of these shapes).  Timed against that one, best of many; the
+    bound leaves twice the largest ratio seen."""
+    def best(p):
+        out, t_min = A.FaFwdPlan(), float("inf")
+        for _ in range(300):
+            t = time.perf_counter()
+            lib.fa_fwd_plan(ctypes.byref(p), CUS, ctypes.byref(out))
+            t_min = min(t_min, time.perf_counter() - t)
+        return t_min
+
+    unsplit = best(contiguous(B=1, H=64, N=4096, D=128, causal=1))
+    mine = best(contiguous(B=1, H=H, N=N, D=D, dtype=A.FA_DTYPE_F16, causal=causal))
+    assert mine < 20 * unsplit, f"{mine * 1e6:.1f} us, unsplit {unsplit * 1e6:.1f}"
