@@ -54,3 +54,40 @@ def test_wide_scores_do_not_double_the_time(fa, causal, N, sigma):
     print(f"  N(0,1): {t1:.4f} ms   N(0,{sigma}^2): {t3:.4f} ms   ratio {t3 / t1:.3f}",
           flush=True)
     assert t3 / t1 < 1.5
+
+
+def _graph_time(fa, q, k, v, launches=50):
+    """us per launch of a captured graph of `launches` forwards: the GPU's
+    time alone, of kernels as short as the call that launches them."""
+    o = torch.empty_like(q)
+    fa.forward(q, k, v, o)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(launches):
+            fa.forward(q, k, v, o)
+    start = torch.cuda.Event(enable_timing=True)
+    stop = torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    for _ in range(8):
+        start.record()
+        graph.replay()
+        stop.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(stop) / launches * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("H,N", [(8, 200), (32, 225), (64, 255)])
+def test_ragged_only_tile_of_a_key_group(fa, H, N):
+    """fp16 non-causal D = 64 with four key tiles: the last group's only tile
+    is the ragged one.  Its masked keys must not send the workgroup to a second
+    pass (1.25x the time of the whole tiles of N = 256 where they did; without,
+    the masking costs a few percent)."""
+    print(f"case perf guard one-step key groups H={H} N={N}", flush=True)
+    t = {}
+    for n in (N, 256):
+        q, k, v = make_qkv(1, H, n, 64, "fp16", seed=case_seed(960), device=DEV)
+        t[n] = _graph_time(fa, q, k, v)
+    print(f"  N={N}: {t[N]:.2f} us   N=256: {t[256]:.2f} us   ratio {t[N] / t[256]:.3f}", flush=True)
+    assert t[N] / t[256] < 1.12
