@@ -102,6 +102,7 @@ void to_kernel_args(const fa_fwd_params* p, fa::KernelArgs* a) {
   a->split.pair = 0;
   a->split.key_groups = 0;
   a->split.head_group = 0;
+  a->split.all_rows = 0;
 }
 
 // Compute units of the calling thread's current device (queried once per

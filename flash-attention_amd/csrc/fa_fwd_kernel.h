@@ -37,6 +37,9 @@ struct SplitPlan {
   // table): each XCD runs its heads in groups of head_group, the q-tiles of
   // a group's heads interleaved longest first; 0 otherwise.
   int32_t head_group;
+  // 1: waves whose rows all lie past N compute like the others (all_rows in
+  // fa_plan.cpp); 0: they only stage tiles.
+  int32_t all_rows;
   // Item i: q-tile (bits 0..15), chunk (16..23), chunk count (24..31).
   uint32_t item[kMaxSplitItems];
   // Item i's first partial slot of its q-tile (items of one q-tile use
@@ -83,6 +86,7 @@ struct FwdArgs {
   int32_t hpx;        // > 0: whole heads per XCD (causal), in groups
   int32_t group_heads, per_group;  // heads, q-tiles of a group
   int32_t half;       // > 0: XCD placement table of 2 half q-tiles per XCD
+  int32_t idle_row;   // waves with rows from here on only stage (D = 64 non-causal, 4 waves)
   FastDiv by_heads, by_qblocks, by_group, by_group_heads;
 };
 

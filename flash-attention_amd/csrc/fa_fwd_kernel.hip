@@ -322,6 +322,8 @@ __device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelA
   const int hg = (lane >> 4) & 1;  // 16-lane group within the half
 
   const int N = args.seq_len;
+  int idle_row = N;
+  if constexpr (D == 64 && !CAUSAL && NW == 4 && !SPLIT) idle_row = args.idle_row;
   // Work item of this workgroup: a q-tile, or with a plan one entry of its
   // table: a chunk of a q-tile's key tiles (split-KV; the plan lists items
   // longest first), or the q-tile of this dispatch position within its XCD
@@ -801,13 +803,13 @@ __device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelA
     constexpr bool OPT = decltype(opt_c)::value;
     // A wave whose rows all lie past N only stages its part of each tile, in
     // a loop of its own (a test in the tile loop cost full grids 1 %): it
-    // leaves the SIMD to the others.  B2 H32 N2100 D128 bf16 163 -> 146 us
-    // (8 waves), causal B8 H12 N300 D128 13.8 -> 13.3; split chunks measured
+    // leaves the SIMD to the others (some grids do without: all_rows).  B2 H32
+    // N2100 D128 bf16 163 -> 146 us (8 waves), causal B8 H12 N300 D128 13.8 -> 13.3; split chunks measured
     // -1.5 % with it (B1 H2 N8192) and go without.  The loop is marked
     // unlikely: as an ordinary branch it made the tile loop of bf16 D = 128
     // 4-wave grids of one to 1.5 workgroups per CU 3...5 % slower, whole tiles
     // included (B1 H20 N1792 42.6 us, 40.5 now), and that of fp16 D = 64 1 %.
-    if (!SPLIT && __builtin_expect(wrow0 >= N, 0)) {
+    if (!SPLIT && __builtin_expect(wrow0 >= idle_row, 0)) {
       for (int u = 0; u < n_steps; ++u) {
         const int t = t_first + TS * u;
         if (t + TS < t_end) issue_tile(t + TS, (u & 1) ^ 1);
@@ -1190,6 +1192,7 @@ int64_t set_order(KernelArgs& a, int BM) {
   else if (a.split.head_group > 0 && a.hpx % a.split.head_group == 0)
     a.group_heads = a.split.head_group;
   a.per_group = a.group_heads * a.n_qblocks;
+  a.idle_row = a.split.all_rows ? INT32_MAX : a.seq_len;
   a.by_heads = make_fast_div(a.heads);
   a.by_qblocks = make_fast_div(a.n_qblocks);
   a.by_group = make_fast_div(a.per_group);

@@ -435,11 +435,26 @@ int key_groups(const KernelArgs& a, int compute_units, const Chunks& ch) {
   return groups;
 }
 
+// Whether waves whose rows all lie past N compute like the others instead of
+// only staging (D = 64 non-causal 4-wave grids).  Only staging frees their SIMD
+// and is 1...2 % faster on most ragged grids, but a CU whose workgroups end
+// early takes two of the last round's where each CU should get one.  Grids
+// with 2.375 to 3 workgroups per CU of at least 800 rows show it: on 102 such
+// grids staging takes 0.98 to 1.11 times as long as computing.  us, staging /
+// computing: bf16 B1 H48 N2016 62.3 / 57.8, H50 N1856 57.2 / 54.3, fp16 H50
+// N1856 61.1 / 57.9.  Below 2.375, above 3 and at shorter rows staging is the
+// faster one, and at D = 128 within 1 %.
+bool all_rows(const KernelArgs& a, int compute_units) {
+  if (a.causal || a.head_dim != 64 || block_rows(a) != 128 || a.seq_len < 800) return false;
+  const int64_t w = (int64_t)a.batch * a.heads * ((a.seq_len + 127) / 128);
+  return 8 * w > 19 * (int64_t)compute_units && w <= 3 * (int64_t)compute_units;
+}
+
 }  // namespace
 
 size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, SplitPlan* plan) {
   plan->n_items = plan->n_slots = plan->n_merge = plan->xcd_heads = plan->pair = 0;
-  plan->head_group = plan->key_groups = 0;
+  plan->head_group = plan->key_groups = plan->all_rows = 0;
   if (compute_units < 1) return 0;
   if (pair_mode(a, compute_units)) {
     plan->pair = 1;
@@ -455,7 +470,10 @@ size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, Spli
     return (size_t)ch.bytes;
   }
   const size_t bytes = plan_xcd_table(a, compute_units, plan);
-  if (plan->n_items == 0) plan->head_group = causal_head_group(a, compute_units, false);
+  if (plan->n_items == 0) {
+    plan->head_group = causal_head_group(a, compute_units, false);
+    plan->all_rows = all_rows(a, compute_units);
+  }
   return bytes;
 }
 

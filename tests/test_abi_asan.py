@@ -4,8 +4,9 @@ fa_api.cpp (the C ABI: validation, status and error strings, workspace
 sizing) and fa_plan.cpp (the split-KV and XCD placement planning, which fills
 fixed-size tables) are compiled with g++ -fsanitize=address and linked with
 the library's own kernel object into a separate libfa_mi355x.so; the CPU tests
-of tests/test_abi.py (every validation branch) and tests/test_split_plan.py
-(plans over the BASELINE configs and a sweep of shapes) then run against that
+of tests/test_abi.py (every validation branch), tests/test_split_plan.py
+(plans over the BASELINE configs and a sweep of shapes) and
+tests/test_split_choice.py (the choice of chunk lengths) then run against that
 build in a child pytest with libasan preloaded.  Any invalid memory access
 makes ASan abort the child with a report.  Needs the kernel object of a
 previous build (flash-attention_amd/_build/fa_fwd_kernel.hip.o).
@@ -42,8 +43,9 @@ def test_host_layer_under_asan(tmp_path):
     env = dict(os.environ, FA_MI355X_LIB=lib, LD_PRELOAD=asan,
                ASAN_OPTIONS="detect_leaks=0:halt_on_error=1:abort_on_error=1")
     child = [sys.executable, "-m", "pytest", "-q", "-x", "-s", "-p", "no:cacheprovider",
-             "-m", "not gpu", "-k", "not runtime",
-             os.path.join(HERE, "test_abi.py"), os.path.join(HERE, "test_split_plan.py")]
+             "-m", "not gpu", "-k", "not runtime and not plan_time",
+             os.path.join(HERE, "test_abi.py"), os.path.join(HERE, "test_split_plan.py"),
+             os.path.join(HERE, "test_split_choice.py")]
     r = subprocess.run(child, capture_output=True, text=True, env=env, cwd=REPO, timeout=600)
     print(r.stdout[-2000:])
     assert "AddressSanitizer" not in r.stderr + r.stdout, (r.stdout + r.stderr)[-4000:]
