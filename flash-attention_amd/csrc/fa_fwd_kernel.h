@@ -116,10 +116,11 @@ int block_rows(const KernelArgs& args);
 // (host code, fa_plan.cpp).
 // Causal grids of 0.75 to 2 q-tiles per CU get pair mode (pair = 1, no
 // items, returns 0) and grids too small for the machine key groups
-// (key_groups, no items, returns 0), with or without a workspace.  Otherwise, with
-// allow_split it may choose split-KV and returns the workspace bytes it
-// needs; without (or when no split pays) it returns 0 and leaves either no
-// plan (n_items = 0) or an XCD placement table (xcd_heads > 0).
+// (key_groups, no items, returns 0), with or without a workspace.  Otherwise,
+// and where it beats two key groups, with allow_split it may choose split-KV
+// and returns the workspace bytes it needs; without (or when no split pays) it
+// returns 0 and leaves either no plan (n_items = 0) or an XCD placement table
+// (xcd_heads > 0).
 size_t plan_split(const KernelArgs& args, int compute_units, bool allow_split, SplitPlan* plan);
 
 // Launches the forward kernel for args (validated by the caller) on stream.

@@ -435,6 +435,19 @@ int key_groups(const KernelArgs& a, int compute_units, const Chunks& ch) {
   return groups;
 }
 
+// Whether a split with chunks of at most S tiles beats two key groups, whose
+// launch is T / 2 steps of the same work as a 256-row tile.  The line is where
+// the measured times cross: of 138 grids below 0.92 the split is 3...18 % faster
+// on those below 0.9 (us, two groups / split: B1 H2 N9032 D64 fp16 69.4 / 60.0,
+// D128 103.1 / 90.4, H3 N7092 D64 bf16 56.2 / 51.7) and 3...5 % slower at 0.919
+// (H4 N5341 D64 43.3 / 45.3).
+bool split_beats_two_groups(const KernelArgs& a, int compute_units, int S) {
+  const int BM = block_rows(a);
+  const ChunkCost split(a, compute_units, BM, (a.seq_len + BM - 1) / BM, S);
+  const int T = (a.seq_len + kKeyTile - 1) / kKeyTile;
+  return split.cost() < 0.9 * 0.5 * T;
+}
+
 // Whether waves whose rows all lie past N compute like the others instead of
 // only staging (D = 64 non-causal 4-wave grids).  Only staging frees their SIMD
 // and is 1...2 % faster on most ragged grids, but a CU whose workgroups end
@@ -463,12 +476,15 @@ size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, Spli
   }
   Chunks ch = average_chunks(a, compute_units);
   plan->key_groups = key_groups(a, compute_units, ch);
-  if (plan->key_groups != 0) return 0;
-  if (allow_split && ch.S > 0) {
+  if (allow_split && ch.S > 0 && plan->key_groups != 4) {
     choose_chunks(a, compute_units, &ch);
-    plan_chunks(a, ch.S, plan);
-    return (size_t)ch.bytes;
+    if (plan->key_groups == 0 || split_beats_two_groups(a, compute_units, ch.S)) {
+      plan->key_groups = 0;
+      plan_chunks(a, ch.S, plan);
+      return (size_t)ch.bytes;
+    }
   }
+  if (plan->key_groups != 0) return 0;
   const size_t bytes = plan_xcd_table(a, compute_units, plan);
   if (plan->n_items == 0) {
     plan->head_group = causal_head_group(a, compute_units, false);

@@ -118,6 +118,23 @@ def test_shorter_launch_is_taken(lib, D, causal):
     assert took == {True, False} or not causal
 
 
+@pytest.mark.parametrize("H,N,D,split", [
+    (3, 7000, 64, True), (3, 7168, 64, True),    # two groups 3...9 % slower than the split
+    (2, 9032, 64, True), (2, 9032, 128, True),
+    (4, 5341, 64, False), (2, 14000, 64, False), (5, 4147, 64, False),  # the split the slower one
+])
+@pytest.mark.parametrize("dtype", [A.FA_DTYPE_F16, A.FA_DTYPE_BF16])
+def test_split_or_two_key_groups(lib, H, N, D, split, dtype):
+    """Non-causal grids of at most one 128-row q-tile per CU run two key groups
+    unless a split's modelled time is clearly lower."""
+    pl = plan(lib, contiguous(B=1, H=H, N=N, D=D, dtype=dtype, causal=0))
+    if split:
+        check_plan(pl, 1, H, N, D, 0)
+        assert pl.workspace_bytes <= SCRATCH
+    else:
+        assert pl.n_items == 0 and pl.block_rows == 128 and pl.workspace_bytes == 0
+
+
 @pytest.mark.parametrize("H,N,D,causal", [
     (1, 32512, 128, 1), (1, 28000, 64, 1), (1, 24000, 128, 1), (2, 24000, 64, 1), (4, 16384, 64, 1),
     (1, 16384, 128, 1), (7, 2500, 128, 1), (8, 2048, 64, 1), (1, 16384, 128, 0),
