@@ -86,8 +86,8 @@ struct FwdArgs {
   int32_t hpx;        // > 0: whole heads per XCD (causal), in groups
   int32_t group_heads, per_group;  // heads, q-tiles of a group
   int32_t half;       // > 0: XCD placement table of 2 half q-tiles per XCD
-  int32_t idle_row;   // waves with rows from here on only stage (D = 64 non-causal, 4 waves)
   FastDiv by_heads, by_qblocks, by_group, by_group_heads;
+  int32_t idle_row;   // waves with rows from here on only stage (D = 64 non-causal, 4 waves)
 };
 
 struct KernelArgs : FwdArgs {
