@@ -274,6 +274,7 @@ fa_status fa_fwd_plan(const fa_fwd_params* p, int32_t compute_units, fa_fwd_plan
   out->xcd_heads = a.split.xcd_heads;
   out->key_halves = a.split.pair ? 2 : a.split.key_groups == 4 ? 4 : 1;
   out->head_group = a.split.head_group;
+  out->reserved = a.split.key_groups;
   for (int i = 0; i < a.split.n_items; ++i) {
     const uint32_t info = a.split.item[i];
     const int qb = (int)(info & 0xffffu), c = (int)((info >> 16) & 0xffu), nch = (int)(info >> 24);

@@ -121,7 +121,7 @@ typedef struct {
 } fa_device_info_t;
 
 /* Work plan of a problem (diagnostic; filled by fa_fwd_plan): split-KV, an XCD
- * placement table, pair mode, or none. */
+ * placement table, pair mode, key groups, or none. */
 #define FA_PLAN_MAX_ITEMS 128
 typedef struct {
   int32_t block_rows;       /* query rows per workgroup (q-tile height) of the kernel */
@@ -132,11 +132,13 @@ typedef struct {
   int32_t key_halves;       /* 2: pair mode (8 waves per q-tile, each half on alternate key
                                tiles, one workgroup per q-tile, no items); 4: the same with
                                four key groups on 64-row q-tiles; 1 otherwise (two groups on
-                               the 128-row q-tiles of small non-causal grids included) */
+                               the 128-row q-tiles of small non-causal grids included: they are
+                               told apart by `reserved`) */
   int32_t head_group;       /* > 0: causal grid without items, B*H a multiple of 8: each XCD
                                runs its heads in groups of this many, the q-tiles of a group
                                interleaved longest first; 0 otherwise */
-  int32_t reserved;         /* 0 */
+  int32_t reserved;         /* key groups outside pair mode: 4 (64-row q-tiles) or 2 (128-row
+                               q-tiles of non-causal grids); 0 otherwise */
   uint64_t workspace_bytes; /* bytes fa_fwd_ws needs (0 when unsplit) */
   /* Split-KV (xcd_heads == 0): work item i (dispatch order, longest first)
    * of every (batch, head) is q-tile q_tile[i], key tiles (64 keys each)
@@ -207,7 +209,8 @@ fa_status fa_fwd_ws_timed(const fa_fwd_params* p, void* workspace, uint64_t work
 fa_status fa_fwd_scratch(const fa_fwd_params* p, void* stream);
 
 /* The work plan fa_fwd_ws would use for *p on a device with
- * `compute_units` CUs (split-KV, an XCD placement table, pair mode, or none).
+ * `compute_units` CUs (split-KV, an XCD placement table, pair mode, key
+ * groups, or none).
  * Host only; touches no GPU. */
 fa_status fa_fwd_plan(const fa_fwd_params* p, int32_t compute_units, fa_fwd_plan_t* out);
 

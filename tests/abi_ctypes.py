@@ -98,6 +98,11 @@ class FaFwdPlan(ctypes.Structure):
         ("head", ctypes.c_int32 * FA_PLAN_MAX_ITEMS),
     ]
 
+    @property
+    def key_groups(self) -> int:
+        """Key groups outside pair mode (4 or 2; 0: none)."""
+        return self.reserved
+
 
 def declared_functions(header: str = HEADER) -> list[str]:
     """Names of the functions declared in the public header."""

@@ -51,7 +51,8 @@ def test_key_groups_vs_oracle(fa, oracle, lib, B, H, N, D, causal, rows, dtype):
     q, k, v = make_qkv(B, H, N, D, dtype, seed=case_seed(1300 + N + D), device=DEV)
     pl, cus = _plan(lib, q, causal)
     if cus == 256:
-        assert pl.block_rows == rows and pl.n_items == 0 and pl.workspace_bytes == 0
+        assert pl.block_rows == rows and pl.key_groups == 256 // rows
+        assert pl.n_items == 0 and pl.workspace_bytes == 0
     o, lse = fa.forward(q, k, v, causal=causal, return_lse=True)
     o2 = fa.forward(q, k, v, causal=causal)  # without an LSE: the same O
     o3 = fa.forward(q, k, v, causal=causal, split_kv=False)
@@ -60,14 +61,17 @@ def test_key_groups_vs_oracle(fa, oracle, lib, B, H, N, D, causal, rows, dtype):
     _check_against_oracle(oracle, q, k, v, o, lse, causal, 1.0 / math.sqrt(D), dtype)
 
 
-@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
-@pytest.mark.parametrize("H,N,D,key,by", [
-    (4, 500, 64, 70, 6.0), (4, 500, 128, 40, 6.0),    # the maximum in another group's first tile
-    (4, 900, 64, 600, 30.0), (4, 900, 128, 600, 30.0),  # far above it, in a later step
-    (20, 900, 128, 600, 30.0),                         # two groups (non-causal)
+@pytest.mark.parametrize("H,N,D,key,by,causal,groups", [
+    # the maximum in another group's first tile
+    (4, 500, 64, 70, 6.0, False, 4), (4, 500, 64, 70, 6.0, True, 4),
+    (4, 500, 128, 40, 6.0, False, 4), (4, 500, 128, 40, 6.0, True, 4),
+    # far above it, in a later step: the group's offset is derived again
+    (8, 900, 64, 600, 30.0, False, 4), (8, 900, 64, 600, 30.0, True, 4),
+    (8, 900, 128, 600, 30.0, False, 4), (8, 900, 128, 600, 30.0, True, 4),
+    (20, 900, 64, 600, 30.0, False, 2), (20, 900, 128, 600, 30.0, False, 2),
 ])
-def test_key_groups_score_jumps_vs_oracle(fa, oracle, H, N, D, key, by, dtype, causal):
+def test_key_groups_score_jumps_vs_oracle(fa, oracle, lib, H, N, D, key, by, causal, groups, dtype):
     """One key scaled far above the others: the groups' offsets lie far
     apart, so all but one group's share of a row vanishes in the combine."""
     print(f"case key groups jump N={N} D={D} key={key} {dtype} causal={causal}", flush=True)
@@ -75,16 +79,20 @@ def test_key_groups_score_jumps_vs_oracle(fa, oracle, H, N, D, key, by, dtype, c
     k = k.clone()
     k[:, :, key] = (k[:, :, key].float() * by).to(k.dtype)
     q, k, v = q.to(DEV), k.to(DEV), v.to(DEV)
+    pl, cus = _plan(lib, q, causal)
+    assert cus != 256 or pl.key_groups == groups
     o, lse = fa.forward(q, k, v, causal=causal, return_lse=True)
     _check_against_oracle(oracle, q, k, v, o, lse, causal, 1.0 / math.sqrt(D), dtype,
                           contract=False)
 
 
-def test_key_groups_strided_views(fa):
+def test_key_groups_strided_views(fa, lib):
     """[B, N, H, D] views and a padded output give the contiguous result; the
     padding is not written."""
     B, H, N, D = 2, 4, 300, 64
     q, k, v = make_qkv(B, H, N, D, "fp16", seed=case_seed(1390), device=DEV)
+    pl, cus = _plan(lib, q, False)
+    assert cus != 256 or pl.key_groups == 4
     ref = fa.forward(q, k, v)
     qs, ks, vs = (t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (q, k, v))
     buf = torch.full((B, H, N, D + 8), 7.0, dtype=q.dtype, device=DEV)

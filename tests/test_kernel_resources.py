@@ -4,7 +4,8 @@ flags (CPU only: hipcc cross-compiles without a GPU).
 
 - Every forward variant fits two waves per SIMD (at most 256 VGPRs, no
   AGPRs), with no scratch and no VGPR spills; the pair-mode variants hold two
-  K/V rings (128 KiB at D = 128, one workgroup per CU).
+  K/V rings (128 KiB at D = 128, one workgroup per CU), the key-group ones one
+  per group.
 - m0 discipline of the K/V staging: the DMA is issued from inline asm that
   sets m0 (the LDS destination) immediately before each
   global_load_lds_dwordx4 and declares m0 clobbered.  The compiler does not
@@ -72,6 +73,20 @@ def test_forward_variants_fit_two_waves_per_simd(device_asm):
     lse_l = [a for a in args.values() if a[6] == "1"]
     assert len(lse_l) == 10 and all(a[1] == "1" and (a[4] == "1" or a[5] == "1") for a in lse_l)
     assert sum("fa_merge_kernel" in n for n, _ in kernels) == 4
+    # key groups <D, BF16, CAUSAL, KG, LSE_L>: four groups causal and not, two
+    # non-causal, bf16 with and without the LSE's sums; a K/V ring per group
+    # (of 32-key tiles for four groups at D = 128), and the flag of the
+    # optimistic pass (all but fp16 causal)
+    kg = {re.search(r"fa_kg_kernelILi(\d+)ELb(\d)ELb(\d)ELi(\d)ELb(\d)E", n).groups(): f
+          for n, f in kernels if "fa_kg_kernel" in n}
+    assert len(kg) == 18 and sum(k[0] == "64" for k in kg) == 9, sorted(kg)
+    assert {(k[2], k[3]) for k in kg} == {("0", "2"), ("0", "4"), ("1", "4")}, sorted(kg)
+    assert not any(k[1] == "0" and k[4] == "1" for k in kg), sorted(kg)
+    for (d, bf16, causal, groups, lse_l), f in kg.items():
+        keys = 32 if d == "128" and groups == "4" else 64
+        ring = int(groups) * 4 * keys * 2 * int(d)
+        opt = bf16 == "1" or causal == "0"
+        assert int(f["group_segment_fixed_size"]) == ring + (4 if opt else 0), (d, bf16, groups)
     # the 16x16x32 kernels <D, BF16, CAUSAL, NW, LSE_L>, D = 64 and 128: fp16
     # and bf16, causal and non-causal, with 4 and 8 waves (no fp16 non-causal
     # 4-wave one at D = 64, which runs the 32x32x16 kernel); bf16 in two

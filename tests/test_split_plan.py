@@ -281,3 +281,19 @@ def test_workspace_bound(lib):
         pl = plan(lib, contiguous(B=1, H=1, N=N, D=128, causal=0))
         assert pl.workspace_bytes <= 128 * 256 * (128 * 4 + 16)
         assert pl.n_slots <= A.FA_PLAN_MAX_ITEMS
+
+
+@pytest.mark.parametrize("H,N,D,causal,groups", [
+    (8, 900, 64, 1, 4), (8, 900, 128, 0, 4), (16, 1024, 64, 0, 4), (8, 193, 64, 0, 4),
+    (20, 900, 64, 0, 2), (17, 1023, 64, 0, 2), (18, 1025, 128, 0, 2), (16, 2048, 128, 0, 2),
+    (64, 1023, 64, 0, 0), (2, 128, 64, 0, 0),   # plain grids
+    (16, 3000, 128, 1, 0), (4, 3000, 128, 1, 0),  # pair mode, split-KV
+])
+def test_key_groups_are_reported(lib, H, N, D, causal, groups):
+    """Two key groups and the plain grid have the same q-tiles: the plan tells
+    them apart."""
+    pl = plan(lib, contiguous(B=1, H=H, N=N, D=D, dtype=A.FA_DTYPE_F16, causal=causal))
+    assert pl.key_groups == groups
+    if groups:
+        assert pl.block_rows == 256 // groups and pl.n_items == 0 and pl.workspace_bytes == 0
+        assert pl.key_halves == (4 if groups == 4 else 1)
