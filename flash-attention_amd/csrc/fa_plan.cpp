@@ -293,49 +293,33 @@ void plan_chunks(const KernelArgs& a, int S, SplitPlan* plan) {
   plan->n_merge = n_merge;
 }
 
-// XCD placement table for a causal 4-wave grid of one round: each XCD
-// (cpx CUs) receives n = heads_per_xcd * nq workgroups, cpx < n <= 2 cpx.
-// Measured dispatch (per-workgroup hardware CU ids): an XCD's k-th
-// workgroup goes to CU slot k mod cpx, so positions k and k + cpx share a
-// CU for k < n - cpx, and positions n - cpx .. cpx - 1 run alone.  Longest
-// first (the default order) pairs the longest q-tile with the (cpx+1)-th
-// longest: at B1 H16 N3000 the 47-tile q-tile shared its CU with a 32-tile
-// one and set the kernel time (66 us).  The table gives the alone
-// positions the longest items and pairs the rest longest with shortest.
-// Grids of 0.75 to 2 q-tiles per CU run in pair mode (plan_split), so the
-// table remains for n = 2 cpx, where no CU runs alone and the pairing is
-// the whole gain.  No q-tile is split and the kernel's arithmetic is that
-// of the plain grid (only the order changes).  Returns 0 (no workspace).
-size_t plan_xcd_table(const KernelArgs& a, int compute_units, SplitPlan* plan) {
+// XCD placement table for a causal 4-wave grid of exactly two q-tiles per CU
+// (below that the grid runs in pair mode): each XCD (cpx CUs) receives 2 cpx
+// workgroups, whole heads.  Measured dispatch (per-workgroup hardware CU ids):
+// an XCD's k-th workgroup goes to CU slot k mod cpx, so positions k and
+// k + cpx share a CU.  Longest first (the default order) pairs the longest
+// q-tile with the (cpx + 1)-th longest; the table pairs long with short: the
+// first half runs longest first, heads interleaved, the second half backwards.
+// No q-tile is split and the kernel's arithmetic is that of the plain grid
+// (only the order changes).  The kernels of the product compute this order
+// (work_item); the table itself is for fa_fwd_plan and the test builds.
+void plan_xcd_table(const KernelArgs& a, int compute_units, SplitPlan* plan) {
   const int BM = block_rows(a);
-  if (!a.causal || BM != 128 || compute_units % 8 != 0) return 0;
+  if (!a.causal || BM != 128 || compute_units % 8 != 0) return;
   const int64_t bh = (int64_t)a.batch * a.heads;
-  if (bh % 8 != 0) return 0;
+  if (bh % 8 != 0) return;
   const int nq = (a.seq_len + BM - 1) / BM;
   const int64_t hpx = bh / 8;
   const int64_t cpx = compute_units / 8;
-  const int64_t n = hpx * nq;
-  if (n <= cpx || n > 2 * cpx || n > kMaxSplitItems) return 0;
-  struct Entry { int len, qb, head; };
-  Entry all[kMaxSplitItems];
-  int cnt = 0;
-  for (int h = 0; h < (int)hpx; ++h)
-    for (int qb = 0; qb < nq; ++qb) all[cnt++] = Entry{q_tile_tiles(a, BM, qb), qb, h};
-  std::stable_sort(all, all + cnt, [](const Entry& x, const Entry& y) {
-    return x.len != y.len ? x.len > y.len : x.qb > y.qb;
-  });
-  // Sorted entry src goes to position: the alone positions take the
-  // longest, then pairs longest-with-shortest.
-  const int m = (int)(n - cpx);
-  const int alone = (int)cpx - m;
-  for (int src = 0; src < cnt; ++src) {
-    const int pos = src < alone ? m + src : (src < alone + m ? src - alone : (int)cpx + (cnt - 1 - src));
-    plan->item[pos] = (uint32_t)all[src].qb | (1u << 24);
-    plan->slot[pos] = (uint32_t)all[src].head;
+  if (hpx * nq != 2 * cpx || hpx * nq > kMaxSplitItems) return;
+  const int n = (int)(hpx * nq);
+  for (int i = 0; i < n; ++i) {
+    const int w = i < n / 2 ? i : n + n / 2 - 1 - i;
+    plan->item[i] = (uint32_t)(nq - 1 - w / (int)hpx) | (1u << 24);
+    plan->slot[i] = (uint32_t)(w % (int)hpx);
   }
-  plan->n_items = cnt;
+  plan->n_items = n;
   plan->xcd_heads = (int)hpx;
-  return 0;
 }
 
 }  // namespace
@@ -485,12 +469,12 @@ size_t plan_split(const KernelArgs& a, int compute_units, bool allow_split, Spli
     }
   }
   if (plan->key_groups != 0) return 0;
-  const size_t bytes = plan_xcd_table(a, compute_units, plan);
+  plan_xcd_table(a, compute_units, plan);
   if (plan->n_items == 0) {
     plan->head_group = causal_head_group(a, compute_units, false);
     plan->all_rows = all_rows(a, compute_units);
   }
-  return bytes;
+  return 0;
 }
 
 }  // namespace fa
