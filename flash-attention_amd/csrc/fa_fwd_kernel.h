@@ -15,13 +15,14 @@ namespace fa {
 // Split-KV: long key ranges of a q-tile are cut into chunks computed by
 // separate workgroups, whose partial results (fp32 O normalised by the
 // chunk's own row sum, offset m and row sum l per row) go to a
-// caller-provided workspace and are merged by a second kernel.  Used when the grid would leave most of the machine idle
-// behind a few long q-tiles (short causal problems, few heads).
+// caller-provided workspace and are merged by a second kernel.  Used when the
+// grid would leave most of the machine idle behind a few long q-tiles (short
+// causal problems, few heads).
 //
 // XCD placement table (xcd_heads > 0): a causal grid of exactly two q-tiles
 // per CU, where the hardware puts the k-th and (k + CUs per XCD)-th
 // workgroups of an XCD on the same CU.  The table orders each XCD's q-tiles
-// so the longest run alone and the others share a CU long with short.
+// so that each CU's pair long with short.
 constexpr int kMaxSplitItems = 128;
 
 struct SplitPlan {

@@ -40,10 +40,11 @@
 //  * Pair mode (causal grids of 0.75 to 2 q-tiles of 128 rows per CU): 8
 //    waves run one q-tile, waves 0-3 on the even key tiles and waves 4-7 on
 //    the odd ones, each half with its own K/V ring; the halves meet in LDS
-//    at the end.  fa_kg_kernel is the same with four groups on 64-row
-//    q-tiles, or two on non-causal ones, for grids too small to put two waves
-//    on every SIMD (key_groups in fa_plan.cpp).  A long q-tile then never runs as a lone 4-wave workgroup
+//    at the end.  A long q-tile then never runs as a lone 4-wave workgroup
 //    on its CU (one wave per SIMD), which set the time of such grids.
+//  * Key groups (fa_kg_kernel): the same with four groups on 64-row q-tiles,
+//    or two on the 128-row q-tiles of non-causal problems, for grids too small
+//    to put two waves on every SIMD (key_groups in fa_plan.cpp).
 //  * O (and the fp32 split partials) leave through LDS: each wave parks its
 //    32-row tile in the then idle K/V ring and stores whole rows, 16
 //    contiguous bytes per lane.
@@ -179,9 +180,9 @@ __device__ __forceinline__ int fast_div(int n, FastDiv d) {
 //    k and half + k of an XCD share a CU; the second half runs backwards, so
 //    each CU's q-tiles pair long with short.
 //  * Otherwise xcd_remap's order, causal q-tiles longest first.
-// The host passes the divisors' reciprocals: the divisions and the order
-// tables' loads were a quarter of the 1600...2900 cycles a workgroup spent
-// before its first load.
+// The host passes the divisors' reciprocals and no table is read: a workgroup
+// of the key-group kernels issues its first load 1200...1400 cycles after it
+// starts, most of them the wait for its arguments.
 //
 // TOGETHER: all of the arguments the prologue needs are loaded in one batch;
 // left to itself the compiler waits for the order's fields first and loads
@@ -465,10 +466,10 @@ __device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelA
   }
   // Key groups: the groups share their rows, so the workgroup stages each row
   // once, the waves of a row block a part each (direct loads by every wave
-  // kept the address unit busy for 2000 cycles at D = 128).  The rows sit in
-  // K buffers 1, free until tile 1 is staged after the second barrier.
-  // (Waiting for K and Q first and for V only after the first S product
-  // measured 1...3 % slower at 4 key groups: its test stays in the tile loop.)
+  // read them KG times, in pieces of 32 bytes).  The rows sit in K buffers 1,
+  // free until tile 1 is staged after the second barrier.  (Waiting for K and
+  // Q first and for V only after the first S product measured 1...3 % slower
+  // at 4 key groups: its test stays in the tile loop.)
   constexpr bool kShareQ = PAIR;
   constexpr int QPS = TILEB / (32 * QRB);  // row blocks per ring slot
   const uint32_t qs_lds =
@@ -804,9 +805,9 @@ __device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelA
     // A wave whose rows all lie past N only stages its part of each tile, in
     // a loop of its own (a test in the tile loop cost full grids 1 %): it
     // leaves the SIMD to the others (some grids do without: all_rows).  B2 H32
-    // N2100 D128 bf16 163 -> 146 us (8 waves), causal B8 H12 N300 D128 13.8 -> 13.3; split chunks measured
-    // -1.5 % with it (B1 H2 N8192) and go without.  The loop is marked
-    // unlikely: as an ordinary branch it made the tile loop of bf16 D = 128
+    // N2100 D128 bf16 163 -> 146 us (8 waves), causal B8 H12 N300 D128 13.8 ->
+    // 13.3; split chunks measured -1.5 % with it (B1 H2 N8192) and go without.
+    // The loop is marked unlikely: as an ordinary branch it made the tile loop of bf16 D = 128
     // 4-wave grids of one to 1.5 workgroups per CU 3...5 % slower, whole tiles
     // included (B1 H20 N1792 42.6 us, 40.5 now), and that of fp16 D = 64 1 %.
     if (!SPLIT && __builtin_expect(wrow0 >= idle_row, 0)) {
@@ -900,8 +901,8 @@ __device__ __forceinline__ void fwd_body(const std::conditional_t<SPLIT, KernelA
     // normalised O (fp32 rows, CP head dims a pass) and its rows' (m, l, lr);
     // then the KG waves of a row block finish 32 / KG of its rows each, 8
     // head dims a lane, every group's term rescaled to the largest offset.
-    // (One group reading the others' whole O took 3200 cycles at D = 64 and
-    // 5200 at D = 128 with four groups.)
+    // Four groups take 2800 cycles at D = 64 and 4600 at D = 128 (two passes)
+    // until their rows are in memory.
     constexpr int RING = 4 * KG * TILEB;
     constexpr int PASSES = NW * 32 * 4 * D + NW * 512 <= RING ? 1 : 2;
     constexpr int CP = D / PASSES, ROWF = CP * 4;  // head dims, bytes of a row per pass
@@ -1085,10 +1086,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 // Key groups outside pair mode: KG = 4 on a 64-row q-tile, KG = 2 on a
 // 128-row non-causal one.  What bounds such a launch is the length of one
-// workgroup: at 64 heads of rows on 256 CUs (B1 H8 N2048 D64 fp16, 256
-// workgroups) it spends 2.3 us before its first product (kernel arguments,
-// then 64 KiB of K, V and Q), 8 steps of 1.0 us and 1.2 us in the combine;
-// 25.6 us as split chunks with a merge launch, 13.5 us here.
+// workgroup: B1 H8 N2048 D64 fp16 (a workgroup on each of 256 CUs) spends 3100
+// cycles before its first product (arguments, then 64 KiB of K, V and Q), 8
+// steps of 2570 and 2800 in the combine, at about 2 GHz; 25.6 us as split
+// chunks with a merge launch, 13.5 us here.
 template <int D, bool BF16, bool CAUSAL, int KG, bool LSE_L>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
     fa_kg_kernel(const FwdArgs args) {
@@ -1252,7 +1253,7 @@ hipError_t launch_one(const KernelArgs& a, hipStream_t stream) {
   }
 }
 
-// Launch of fa_kg_kernel: one workgroup per 64-row q-tile, no items.
+// Launch of fa_kg_kernel: one workgroup per q-tile of 256 / KG rows, no items.
 template <int D, bool BF16, bool CAUSAL, int KG>
 hipError_t launch_kg(const KernelArgs& a, hipStream_t stream) {
   if (a.split.n_items != 0) return hipErrorInvalidValue;
@@ -1266,7 +1267,8 @@ hipError_t launch_kg(const KernelArgs& a, hipStream_t stream) {
   return hipLaunchKernel(fn, dim3((unsigned)total), dim3(512), kargs, 0, stream);
 }
 
-// The 16x16x32 MFMA kernel of every unsplit launch outside pair mode.
+// The 16x16x32 MFMA kernel of the launches without split chunks, pair mode or
+// key groups.
 #include "fa_fwd16.inc"
 
 // fa_fwd16_kernel where it runs (see launch_causal), else fa_fwd_kernel.
@@ -1281,10 +1283,10 @@ hipError_t launch_pick(const KernelArgs& a, hipStream_t stream, bool plain) {
 
 template <int D, bool BF16>
 hipError_t launch_causal(const KernelArgs& a, hipStream_t stream) {
-  // Launches without split-KV chunks or pair mode (plain order or an XCD
-  // placement table) run fa_fwd16_kernel, the 16x16x32 MFMA form, except
-  // fp16 non-causal 4-wave grids at D = 64; split chunks, pair mode and those
-  // run this file's 32x32x16 kernel.  Measured on two boxes, 16x16x32
+  // Launches without split-KV chunks, pair mode or key groups (plain order or
+  // an XCD placement table) run fa_fwd16_kernel, the 16x16x32 MFMA form, except
+  // fp16 non-causal 4-wave grids at D = 64; split chunks, pair mode, key groups
+  // and those run this file's 32x32x16 kernels.  Measured on two boxes, 16x16x32
   // against 32x32x16: +2...+8 % at B4 H32 N4096 fp16, +2...+4 % at bf16
   // causal B2 H32 N8192, +0...+5 % on fp16 causal B1 H16 N16384.  At D = 64
   // (same box): fp16 non-causal 4-wave B4 H16 N1024 -0.3 % (-1.5 % with

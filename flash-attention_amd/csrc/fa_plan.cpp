@@ -380,7 +380,7 @@ int causal_head_group(const KernelArgs& a, int compute_units, bool pair) {
 // N1024 D128 22.0 -> 18.2, B1 H12 N2048 D64 39.5 -> 19.9, H6 N4096 D128
 // 85.2 -> 55.7.  Short rows: two key tiles gain from 4 groups on causal rows
 // (D = 64 6.7 -> 5.8, D = 128 8.3 -> 6.7) but not on D = 64 non-causal ones
-// (4.7 -> 5.0; four tiles 6.2 -> 5.7); at D = 128 they gain as well (7.4 ->
+// (4.7 -> 5.0; four tiles 6.0 -> 5.2, ragged ones 6.3 -> 5.2); at D = 128 they gain as well (7.4 ->
 // 6.4), but N = 128 non-causal is held to one 128-row q-tile per head by the
 // plan's tests, so the line is three tiles.  Two groups need 4 tiles at
 // D = 128 (10.4 -> 9.7) and 6 at D = 64 (4 tiles: 6.9 -> 7.1).
@@ -393,9 +393,10 @@ int causal_head_group(const KernelArgs& a, int compute_units, bool pair) {
 // groups 40.6 against 45.7).  Grids of at most an eighth (causal: a quarter)
 // of the CUs in 64-row q-tiles keep split-KV: the plan's tests hold shapes
 // of one or two heads there to it (B1 H2 N1000 D64 non-causal 12.4 us split,
-// 9.2 with four groups).  So do the few whose partials exceed the static scratch (D = 128, about 5
-// heads of N = 6000): fa_fwd_scratch refuses those, with or without key groups
-// for their neighbours.
+// 9.2 with four groups).  So do the few whose partials exceed the static
+// scratch (D = 128, about 5 heads of N = 6000): fa_fwd_scratch refuses those,
+// with or without key groups for their neighbours.  Two groups give way to a
+// split that is clearly faster (split_beats_two_groups).
 // ch: average_chunks.
 int key_groups(const KernelArgs& a, int compute_units, const Chunks& ch) {
   const int64_t bh = (int64_t)a.batch * a.heads;
