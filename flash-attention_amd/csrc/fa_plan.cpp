@@ -436,7 +436,7 @@ bool split_beats_two_groups(const KernelArgs& a, int compute_units, int S) {
 // Whether waves whose rows all lie past N compute like the others instead of
 // only staging (D = 64 non-causal 4-wave grids).  Only staging frees their SIMD
 // and is 1...2 % faster on most ragged grids, but a CU whose workgroups end
-// early takes two of the last round's where each CU should get one.  Grids
+// early takes two of the remaining ones where each CU should get one.  Grids
 // with 2.375 to 3 workgroups per CU of at least 800 rows show it: on 102 such
 // grids staging takes 0.98 to 1.11 times as long as computing.  us, staging /
 // computing: bf16 B1 H48 N2016 62.3 / 57.8, H50 N1856 57.2 / 54.3, fp16 H50

@@ -4,7 +4,7 @@ to a launch and leaves the results as they are, so a small program reads it
 from fa::plan_split itself.
 
 Only staging made D = 64 non-causal grids of 2.375 to 3 workgroups per CU up to
-11 % slower: CUs whose workgroups ended early took two of the last round's."""
+11 % slower: CUs whose workgroups ended early took two of the remaining ones."""
 from __future__ import annotations
 
 import os
